@@ -41,7 +41,19 @@ struct GemvArgs {
 };
 
 constexpr int kGemvWaves = 8;
-constexpr int kGemmMinM = 56;  // rows of x from which the matrix-core GEMM runs (measured crossover)
+// Rows of x from which the K-split matrix-core GEMM runs, for K up to
+// kKsMaxK.  (q/k/v of 2048, 512 and 512 rows, GEMV / K-split: M = 2 3.7 / 3.8
+// us, M = 3 5.0 / 3.9, M = 16 10.1 / 3.9.)
+constexpr int kKsMinM = 3;
+constexpr int kKsMaxK = 4096;  // (its LDS scale table's groups)
+// Beyond that K, rows of x from which the tile GEMM runs instead of the GEMV
+// (measured crossover)
+constexpr int kGemmMinM = 56;
+// Rows of x from which the tile GEMM runs for any K.  (q/k/v, K-split / tile:
+// M = 512 17.4 / 24.4 us, 768 26.1 / 24.9; out_proj 768 20.6 / 27.7, 1024
+// 25.5 / 28.8.  The line does not depend on the rows of W, so that one
+// matrix gives the same bits alone and in a q/k/v launch.)
+constexpr int kTileMinM = 769;
 
 // nibbles sh..sh+3 and sh+16..sh+19 of w as fp16 (nibble - 8), exact
 __device__ __forceinline__ f16x2 nib_pair(uint32_t w, int sh) {
@@ -254,29 +266,74 @@ __device__ __forceinline__ f16x8 nib8(uint32_t u) {
   return r;
 }
 
-// weight row of global column col (clamped), across the up to 3 matrices
-struct ColRef {
-  const uint8_t* packed;
-  const uint16_t* scales;
-};
-__device__ __forceinline__ ColRef col_ref(const GemvArgs& a, int col, int K) {
-  int n = col < a.rows ? col : a.rows - 1, mi = 0;
-  if (n >= a.mat[0].N) {
-    n -= a.mat[0].N;
-    mi = 1;
-    if (n >= a.mat[1].N) {
-      n -= a.mat[1].N;
-      mi = 2;
-    }
-  }
-  const uint8_t* pk = mi == 0 ? a.mat[0].packed : (mi == 1 ? a.mat[1].packed : a.mat[2].packed);
-  const uint16_t* sc = mi == 0 ? a.mat[0].scales : (mi == 1 ? a.mat[1].scales : a.mat[2].scales);
-  return ColRef{pk + (size_t)n * (K >> 1), sc + (size_t)n * (K >> 7)};
+// A pointer of the kernel arguments as a scalar value.  (Left visible, the
+// per-column choice between the three matrices' pointers below becomes a
+// choice of address and one vector load from the argument segment: a memory
+// round trip before the first operand load and another before the outputs.)
+template <class T>
+__device__ __forceinline__ T* arg_ptr(T* p) {
+  uint64_t v = (uint64_t)p;
+  asm("" : "+s"(v));
+  return (T*)v;
 }
+template <class T>
+__device__ __forceinline__ T* pick(int mi, T* p0, T* p1, T* p2) {
+  T *a = arg_ptr(p0), *b = arg_ptr(p1), *c = arg_ptr(p2);
+  return mi == 0 ? a : (mi == 1 ? b : c);
+}
+
+// global column col (clamped) across the up to 3 matrices: matrix, row of it
+struct ColRef {
+  int mi, n;
+};
+__device__ __forceinline__ ColRef col_ref(const GemvArgs& a, int col) {
+  const int c = col < a.rows ? col : a.rows - 1, n0 = a.mat[0].N, n1 = n0 + a.mat[1].N;
+  const int mi = c >= n1 ? 2 : (c >= n0 ? 1 : 0);
+  return ColRef{mi, c - (mi == 2 ? n1 : (mi == 1 ? n0 : 0))};
+}
+__device__ __forceinline__ const uint8_t* col_packed(const GemvArgs& a, ColRef c, int K) {
+  return pick(c.mi, a.mat[0].packed, a.mat[1].packed, a.mat[2].packed) + (size_t)c.n * (K >> 1);
+}
+__device__ __forceinline__ const uint16_t* col_scales(const GemvArgs& a, ColRef c, int K) {
+  return pick(c.mi, a.mat[0].scales, a.mat[1].scales, a.mat[2].scales) + (size_t)c.n * (K >> 7);
+}
+
+// What a launch does with its sums: store them (fp32), add them to y (fp32:
+// out_proj into the residual), or store them as fp16 (q/k/v).
+enum GemmOut { kOutF32, kOutAdd, kOutF16 };
+
+// The output column of a lane: rows m of it at p + m * N
+template <int kOut>
+struct OutCol {
+  float* y32;
+  uint16_t* y16;
+  int N;
+  __device__ __forceinline__ OutCol(const GemvArgs& a, int col) {
+    const ColRef c = col_ref(a, col);
+    N = c.mi == 0 ? a.mat[0].N : (c.mi == 1 ? a.mat[1].N : a.mat[2].N);
+    if constexpr (kOut == kOutF16)
+      y16 = pick(c.mi, a.mat[0].y16, a.mat[1].y16, a.mat[2].y16) + c.n;
+    else
+      y32 = pick(c.mi, a.mat[0].y32, a.mat[1].y32, a.mat[2].y32) + c.n;
+  }
+  // the residual at row m (read ahead of the sums, so the reads of a lane's
+  // rows are in flight together)
+  __device__ __forceinline__ float old(int m) const {
+    if constexpr (kOut == kOutAdd) return y32[(size_t)m * N];
+    return 0.f;
+  }
+  __device__ __forceinline__ void put(int m, float v, float yold) const {
+    if constexpr (kOut == kOutF16)
+      y16[(size_t)m * N] = f2h(v);
+    else
+      y32[(size_t)m * N] = kOut == kOutAdd ? yold + v : v;
+  }
+};
 
 // grid = (ceil(rows / 128), ceil(M / 128)), block = 64 * kGemmWaves.
 // (Giving each XCD a contiguous run of tiles, so its L2 sees a few row
 // blocks of X rather than all, measured no faster.)
+template <int kOut>
 __global__ __launch_bounds__(64 * kGemmWaves) void k_gemm_int4(GemvArgs a) {
   __shared__ __attribute__((aligned(16))) uint8_t ring[kRing * kSlot];
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
@@ -297,9 +354,9 @@ __global__ __launch_bounds__(64 * kGemmWaves) void k_gemm_int4(GemvArgs a) {
   //   W: wave w fills columns 16 w .. +15; lane l takes column 16 w + (l >> 2),
   //      physical chunk l & 3
   const int wcol = 16 * w + (l >> 2);
-  const uint8_t* wsrc = col_ref(a, r0 + wcol, K).packed + 16 * ((l & 3) ^ ((wcol >> 2) & 3));
+  const uint8_t* wsrc = col_packed(a, col_ref(a, r0 + wcol), K) + 16 * ((l & 3) ^ ((wcol >> 2) & 3));
   //   scales: waves 0, 1 fill columns 64 w + l; the others the drop area
-  const uint16_t* ssrc = col_ref(a, r0 + 64 * (w & 1) + l, K).scales;
+  const uint16_t* ssrc = col_scales(a, col_ref(a, r0 + 64 * (w & 1) + l), K);
   const int sdst = kXSlot + kWSlot + (w < 2 ? 256 * w : 512);
   auto issue = [&](int g) {
     uint8_t* slot = ring + (g % kRing) * kSlot;
@@ -363,38 +420,250 @@ __global__ __launch_bounds__(64 * kGemmWaves) void k_gemm_int4(GemvArgs a) {
 #pragma unroll
         for (int e = 0; e < 4; e++) C[i][j][e] = __builtin_fmaf(P[i][j][e], scl[j], C[i][j][e]);
   }
-  // outputs: lane holds rows 4q + e of tile i, column n16 of tile j
+  // outputs: lane holds rows 4q + e of tile i, column n16 of tile j; the
+  // residual of a column's 16 rows is read before the first is stored
+  // (rows past M read the last one)
 #pragma unroll
   for (int j = 0; j < 2; j++) {
     const int col = r0 + 32 * wn + 16 * j + n16;
-    if (col >= a.rows) continue;
-    int n = col, mi = 0;
-    if (n >= a.mat[0].N) {
-      n -= a.mat[0].N;
-      mi = 1;
-      if (n >= a.mat[1].N) {
-        n -= a.mat[1].N;
-        mi = 2;
-      }
-    }
-    float* y32 = mi == 0 ? a.mat[0].y32 : (mi == 1 ? a.mat[1].y32 : a.mat[2].y32);
-    uint16_t* y16 = mi == 0 ? a.mat[0].y16 : (mi == 1 ? a.mat[1].y16 : a.mat[2].y16);
-    const int N = mi == 0 ? a.mat[0].N : (mi == 1 ? a.mat[1].N : a.mat[2].N);
+    const OutCol<kOut> o(a, col);
+    float yo[4][4];
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         const int m = m0 + 64 * wm + 16 * i + 4 * q + e;
-        if (m >= a.M) continue;
-        const size_t o = (size_t)m * N + n;
-        const float v = C[i][j][e];
-        if (y32) y32[o] = a.add ? y32[o] + v : v;
-        if (y16) y16[o] = f2h(v);
+        yo[i][e] = o.old(m < a.M ? m : a.M - 1);
       }
+    if (col < a.rows) {
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int m = m0 + 64 * wm + 16 * i + 4 * q + e;
+          if (m < a.M) o.put(m, C[i][j][e], yo[i][e]);
+        }
+    }
   }
   // (the last two DMAs refetch the final group into free slots; let them
   // land before the workgroup's LDS is released)
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+}
+
+// ---------------------------------------------------------------- K-split GEMM
+// A few to about a thousand rows of x (short prompts, chat turns): too few
+// 128 x 128 tiles to fill the chip, and each tile's 16 scale groups a serial
+// chain.  Here a workgroup computes a (16 kMT) x (16 kNT) tile with 8 waves
+// that split K: wave w takes the scale groups w, w + 8, .. (two of them at
+// K = 2048), alone, with no barrier before the end.
+//   A lane's 16-byte loads reach 64 bytes a clock only when 4 neighbouring
+//   lanes read 64 contiguous bytes (measured: 256 KB into one compute unit in
+//   1.2 us; in the MFMA operand's own order, neighbouring lanes in different
+//   rows, 6.2 us), so both operands are fetched 4 lanes to a row's 64 bytes
+//   and change lanes afterwards:
+//     x     by DMA into the wave's own LDS: instruction (i, q) brings the k =
+//           32q .. 32q + 31 of row tile i's 16 rows, row r's 16-byte piece s
+//           at s ^ (r >> 2) ^ (q & 1), so that the 16 rows of an operand read
+//           take distinct banks.  Read back as whole operands, after which
+//           the next group's DMA goes out, ahead of this group's products;
+//     W     into registers, then to operand order by ds_bpermute.
+//   The scales of the tile's columns are fetched once, group-fastest as they
+//   lie in memory, into an LDS table.
+// As in the tile kernel, a group's products accumulate from zero and are added
+// in fp32 with the column's scale.  The 8 waves' partial tiles meet in LDS and
+// are added in wave order, so an output's bits do not depend on the tile shape.
+constexpr int kKsWaves = 8;
+
+// grid = (ceil(rows / (16 kNT)), ceil(M / (16 kMT))), block = 512; K <= kKsMaxK
+template <int kOut, int kMT, int kNT>
+__global__ __launch_bounds__(64 * kKsWaves) void k_gemm_int4_ks(GemvArgs a) {
+  static_assert(kNT <= 4, "a wave's partial tile takes its x slot's place");
+  __shared__ __attribute__((aligned(16))) uint8_t xs[kKsWaves * kMT * 4096];
+  __shared__ float ssc[kKsMaxK / 128][16 * kNT];
+  const int tid = threadIdx.x, l = tid & 63, n16 = l & 15, q = l >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m0 = blockIdx.y * 16 * kMT, r0 = blockIdx.x * 16 * kNT;
+  const int K = a.K, ng = K >> 7;
+  uint8_t* xw = xs + w * kMT * 4096;
+  const uint8_t* wp[kNT];
+#pragma unroll
+  for (int j = 0; j < kNT; j++)
+    wp[j] = col_packed(a, col_ref(a, r0 + 16 * j + (l >> 2)), K) + 16 * (l & 3);
+  const uint8_t* xp[kMT][2];  // the row's 64-byte pieces of even and odd q
+#pragma unroll
+  for (int i = 0; i < kMT; i++) {
+    const int r = l >> 2, m = m0 + 16 * i + r;
+    const uint8_t* row = (const uint8_t*)(a.x + (size_t)(m < a.M ? m : a.M - 1) * K);
+    xp[i][0] = row + 16 * ((l & 3) ^ (r >> 2));
+    xp[i][1] = row + 16 * ((l & 3) ^ (r >> 2) ^ 1);
+  }
+  u32x4 wq[kNT], wn[kNT];
+  auto load_w = [&](int g, u32x4 (&o)[kNT]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < kNT; j++) o[j] = *(const u32x4*)(wp[j] + 64 * (size_t)g);
+  };
+  auto load_x = [&](int g) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < kMT; i++)
+#pragma unroll
+      for (int c = 0; c < 4; c++)
+        __builtin_amdgcn_global_load_lds((gbl_void_t*)(xp[i][c & 1] + 256 * (size_t)g + 64 * c),
+                                         (lds_void_t*)(xw + (4 * i + c) * 1024), 16, 0, 0);
+  };
+  const int gf = w < ng ? w : 0;
+  load_w(gf, wq);
+  // the output tiles this wave adds up at the end (w, w + 8, ..): their
+  // residual goes out with the operands
+  constexpr int kTiles = kMT * kNT, kPer = (kTiles + kKsWaves - 1) / kKsWaves;
+  float yo[kPer][4];
+#pragma unroll
+  for (int u = 0; u < kPer; u++) {
+    const int t = w + kKsWaves * u < kTiles ? w + kKsWaves * u : 0;
+    const OutCol<kOut> o(a, r0 + 16 * (t % kNT) + n16);
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int m = m0 + 16 * (t / kNT) + 4 * q + e;
+      yo[u][e] = o.old(m < a.M ? m : a.M - 1);
+    }
+  }
+  load_x(gf);
+  // the scale table: 16 neighbouring threads read a column's 16 groups
+  for (int g0 = 0; g0 < ng; g0 += 16)
+#pragma unroll
+    for (int e = tid; e < 256 * kNT; e += 64 * kKsWaves) {
+      const int c = e >> 4, g = g0 + (e & 15);
+      if (g < ng) ssc[g][c] = h2f(col_scales(a, col_ref(a, r0 + c), K)[g]);
+    }
+  f32x4 C[kMT][kNT];
+#pragma unroll
+  for (int i = 0; i < kMT; i++)
+#pragma unroll
+    for (int j = 0; j < kNT; j++) C[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  __syncthreads();  // the scale table is in
+  auto step = [&](int g, const u32x4 (&cur)[kNT], u32x4 (&nxt)[kNT]) __attribute__((always_inline)) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this group's x and W
+    // lane (n16, q)'s chunk q of column n16 was loaded by lane 4 n16 + q
+    u32x4 wt[kNT];
+#pragma unroll
+    for (int j = 0; j < kNT; j++)
+#pragma unroll
+      for (int s = 0; s < 4; s++)
+        wt[j][s] = (uint32_t)__builtin_amdgcn_ds_bpermute(16 * n16 + 4 * q, (int)cur[j][s]);
+    float scl[kNT];
+#pragma unroll
+    for (int j = 0; j < kNT; j++) scl[j] = ssc[g][16 * j + n16];
+    f16x8 A[kMT][4];
+#pragma unroll
+    for (int i = 0; i < kMT; i++)
+#pragma unroll
+      for (int s = 0; s < 4; s++)
+        A[i][s] = *(const f16x8*)(xw + (4 * i + q) * 1024 + 64 * n16 + 16 * (s ^ (n16 >> 2) ^ (q & 1)));
+    if (g + kKsWaves < ng) {
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the slot is read
+      __builtin_amdgcn_sched_barrier(0);
+      load_w(g + kKsWaves, nxt);
+      load_x(g + kKsWaves);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int j = 0; j < kNT; j++) {
+      f32x4 P[kMT];
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        const f16x8 B = nib8(wt[j][s]);
+#pragma unroll
+        for (int i = 0; i < kMT; i++)
+          P[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[i][s], B, s == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : P[i],
+                                                        0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < kMT; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) C[i][j][e] = __builtin_fmaf(P[i][e], scl[j], C[i][j][e]);
+    }
+  };
+  for (int g = w; g < ng; g += 2 * kKsWaves) {
+    step(g, wq, wn);
+    if (g + kKsWaves < ng) step(g + kKsWaves, wn, wq);
+  }
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // (a wave without groups: its fetch done)
+  f32x4* part = (f32x4*)xs;            // [wave, 256 kMT apart][tile][lane] of 4 rows x 1 column
+#pragma unroll
+  for (int i = 0; i < kMT; i++)
+#pragma unroll
+    for (int j = 0; j < kNT; j++) part[w * kMT * 256 + (i * kNT + j) * 64 + l] = C[i][j];
+  __syncthreads();
+  // the partial tiles in wave order; lane holds rows 4q .. 4q + 3 of column n16
+#pragma unroll
+  for (int u = 0; u < kPer; u++) {
+    const int t = w + kKsWaves * u;
+    if (t >= kTiles) break;
+    const int col = r0 + 16 * (t % kNT) + n16;
+    const OutCol<kOut> o(a, col);
+    f32x4 pv[kKsWaves];
+#pragma unroll
+    for (int k = 0; k < kKsWaves; k++) pv[k] = part[k * kMT * 256 + t * 64 + l];
+    f32x4 v = pv[0];
+#pragma unroll
+    for (int k = 1; k < kKsWaves; k++) v += pv[k];
+    if (col < a.rows) {
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int m = m0 + 16 * (t / kNT) + 4 * q + e;
+        if (m < a.M) o.put(m, v[e], yo[u][e]);
+      }
+    }
+  }
+}
+
+template <int kOut, int kMT, int kNT>
+static void ks_launch(const GemvArgs& a, hipStream_t s) {
+  hipLaunchKernelGGL((k_gemm_int4_ks<kOut, kMT, kNT>),
+                     dim3((unsigned)((a.rows + 16 * kNT - 1) / (16 * kNT)),
+                          (unsigned)((a.M + 16 * kMT - 1) / (16 * kMT))),
+                     dim3(64 * kKsWaves), 0, s, a);
+}
+
+// The K-split kernel's tile shape: the one of least expected time, c (the time
+// of one round of workgroups less the 2.2 us of an empty launch, measured) times
+// the rounds.  A 4-row-tile workgroup has a compute unit to itself (128 KB of
+// LDS), so its rounds are whole; the smaller ones overlap from one round into
+// the next.  (Launches of 2048 rows of W, in us, chosen shape first: M = 16:
+// 1x1 4.2, 2x2 5.7; 64: 1x2 5.1, 2x2 5.7, 1x1 5.7; 128: 2x2 6.0, 4x4 11.3,
+// 1x1 8.9; 300: 4x3 9.9, 2x2 11.5, 4x4 12.0, 1x1 16.9; 512: 4x4 13.4, 2x2
+// 14.0, 1x1 25.0.)
+struct KsShape {
+  int mt, nt;
+  float c;
+};
+constexpr KsShape kKsShapes[] = {{1, 1, 1.7f}, {1, 2, 2.5f}, {2, 2, 3.4f}, {2, 3, 4.4f},
+                                 {2, 4, 5.4f}, {4, 3, 7.2f}, {4, 4, 9.3f}};
+
+static float ks_time(const KsShape& k, int M, int rows) {
+  const int wgs = ((rows + 16 * k.nt - 1) / (16 * k.nt)) * ((M + 16 * k.mt - 1) / (16 * k.mt));
+  const float r = (float)wgs / 256.0f;
+  return k.c * (r <= 1.0f ? 1.0f : (k.mt == 4 ? (float)((wgs + 255) / 256) : r));
+}
+
+// the matrix-core kernels, by the launch's output form
+template <int kOut>
+static void gemm_launch(const GemvArgs& a, hipStream_t s) {
+  if (a.M < kTileMinM && a.K <= kKsMaxK) {
+    int b = 0;
+    for (int i = 1; i < (int)(sizeof(kKsShapes) / sizeof(kKsShapes[0])); i++)
+      if (ks_time(kKsShapes[i], a.M, a.rows) < ks_time(kKsShapes[b], a.M, a.rows)) b = i;
+    switch (10 * kKsShapes[b].mt + kKsShapes[b].nt) {
+      case 11: return ks_launch<kOut, 1, 1>(a, s);
+      case 12: return ks_launch<kOut, 1, 2>(a, s);
+      case 22: return ks_launch<kOut, 2, 2>(a, s);
+      case 23: return ks_launch<kOut, 2, 3>(a, s);
+      case 24: return ks_launch<kOut, 2, 4>(a, s);
+      case 43: return ks_launch<kOut, 4, 3>(a, s);
+      case 44: return ks_launch<kOut, 4, 4>(a, s);
+    }
+  }
+  hipLaunchKernelGGL(k_gemm_int4<kOut>, dim3((unsigned)((a.rows + kTile - 1) / kTile),
+                     (unsigned)((a.M + kTile - 1) / kTile)), dim3(64 * kGemmWaves), 0, s, a);
 }
 
 template <int kM>
@@ -416,9 +685,13 @@ static void gemv_launch(const GemvArgs& a, hipStream_t s) {
 static int gemv_run(GemvArgs& a, void* stream) {
   a.rows = a.mat[0].N + a.mat[1].N + a.mat[2].N;
   hipStream_t s = (hipStream_t)stream;
-  if (a.M >= kGemmMinM) {
-    hipLaunchKernelGGL(k_gemm_int4, dim3((unsigned)((a.rows + kTile - 1) / kTile),
-                       (unsigned)((a.M + kTile - 1) / kTile)), dim3(64 * kGemmWaves), 0, s, a);
+  if (a.M >= (a.K <= kKsMaxK ? kKsMinM : kGemmMinM)) {
+    if (a.mat[0].y16)
+      gemm_launch<kOutF16>(a, s);
+    else if (a.add)
+      gemm_launch<kOutAdd>(a, s);
+    else
+      gemm_launch<kOutF32>(a, s);
   } else if (a.M == 1)
     gemv_launch<1>(a, s);
   else if (a.M == 2)

@@ -110,3 +110,25 @@ def test_qkv_proj_int4(orc, cia, dev, M, seed):
         ref, ab = orc.gemv_int4(x, *W[n], want_absum=True)
         _check(got16.astype(np.float32), ref, ab, n,
                extra=np.abs(ref) * 2.0 ** -11 + 2.0 ** -25)
+
+
+# The K-split GEMM (3 to 768 rows of x, K up to 4096) at the edges of its
+# dispatch and tiles: first and last M, one row past a tile, rows of W that
+# end inside a tile, fewer groups than waves (K = 128, 384), a second and a
+# partial third pass over the groups (K = 1152, 2176), the largest K and the
+# first beyond it, and M on both sides of each shape's choice.
+KSPLIT = [(100, 128, 3, 20), (130, 384, 16, 21), (47, 1152, 17, 22), (200, 2176, 33, 23),
+          (48, 4096, 65, 24), (48, 4224, 40, 25), (2000, 256, 130, 26), (2048, 128, 300, 27),
+          (2050, 384, 511, 28), (33, 256, 768, 29), (33, 256, 769, 30)]
+
+
+@pytest.mark.parametrize("N,K,M,seed", KSPLIT)
+def test_gemm_ksplit(orc, cia, dev, N, K, M, seed):
+    test_gemv_int4(orc, cia, dev, N, K, M, "normal", seed)
+
+
+@pytest.mark.parametrize("M,seed", [(2, 31), (16, 32), (40, 33), (300, 34)])
+def test_qkv_ksplit_bits(orc, cia, dev, M, seed):
+    """q/k/v in one launch have the bits of the three matrices alone,
+    whatever tile shapes the launches take."""
+    test_qkv_proj_int4(orc, cia, dev, M, seed)
