@@ -180,11 +180,21 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill_mfma(PrefillArgs a) {
 
 using namespace cia;
 
-// Internal entry used by cia_attention_fused once its arguments are checked.
+extern "C" __attribute__((visibility("hidden"))) int cia_prefill_split_wins(int S, int past);
+extern "C" __attribute__((visibility("hidden"))) int cia_prefill_split(
+    const uint16_t* q, const uint8_t* kc8, const uint8_t* vc8, const uint16_t* ksc,
+    const uint16_t* vsc, const uint16_t* ktail, const uint16_t* vtail, int committed,
+    uint16_t* out, int S, int past, float scale, void* stream);
+
+// Internal entry used by cia_attention_fused once its arguments are checked:
+// the block kernel, or prefill_split.hip's where that is the faster.
 extern "C" __attribute__((visibility("hidden"))) int cia_prefill_mfma(
     const uint16_t* q, const uint8_t* kc8, const uint8_t* vc8, const uint16_t* ksc,
     const uint16_t* vsc, const uint16_t* ktail, const uint16_t* vtail, int committed,
     uint16_t* out, int S, int past, float scale, void* stream) {
+  if (cia_prefill_split_wins(S, past))
+    return cia_prefill_split(q, kc8, vc8, ksc, vsc, ktail, vtail, committed, out, S, past, scale,
+                             stream);
   const int nblk = (S + kPfQ - 1) / kPfQ;
   PrefillArgs pa{q, kc8, vc8, ksc, vsc, ktail, vtail, committed, out, S, past,
                  scale * kPfLog2e, nblk};

@@ -190,10 +190,11 @@ __device__ __forceinline__ float pf_remax(const f32x4 (&S)[4], float c, bool fir
       const bool out = kMask && key0 + 16 * kt + i > qpos;
       cm = __builtin_fmaxf(cm, out ? -__builtin_inff() : S[kt][i]);
     }
-  // finite on a first tile (key 0 is never masked); c > 0
+  // -inf where every key of the tile is masked (a first tile too when it does
+  // not hold key 0); c > 0
   const float mt = pf_colmax(cm) * c;
   if (first) {
-    m = mt;
+    m = __builtin_fmaxf(mt, -1e30f);
   } else if (mt > m) {
     const float corr = __builtin_amdgcn_exp2f(m - mt);
     m = mt;

@@ -167,6 +167,47 @@ def test_prefill_matrix_cores(orc, cia, dev, S, past, outliers, zero_group):
     assert_close_f16(_u16(out), r32)
 
 
+@pytest.mark.parametrize("S,past", [
+    (1, 200), (5, 0), (16, 48), (17, 640), (33, 1337), (128, 40), (129, 1340), (130, 2700),
+    (3000, 100)])
+def test_prefill_shapes(orc, cia, dev, S, past):
+    """attention_fused at the edges of its choice of kernel and of the split
+    kernel's tiles: fewer key tiles than waves, keys in the tail alone, query
+    tiles that end inside 16 and 32, each wave count, and the block kernel
+    with a history and a ragged last block.  Tail rows past the last token
+    hold NaN, which must not reach the outputs; a second call with the tail
+    rows visible as committed keys only (committed > past + S) must not read
+    past the queries' own keys."""
+    from cuda_inf_amd import kernels as K
+    from cuda_inf_amd.layer import AttnLayer
+    from cuda_inf_amd.workload import qkv
+    L = AttnLayer(past + S + 128, nsplit=16, device=dev)
+    L.ktail.fill_(float("nan"))
+    L.vtail.fill_(float("nan"))
+    ref = orc.Group64Cache(past + S + 128)
+    _, k0, v0 = qkv(past + S, seed=13, device="cpu", outliers=True)
+    q, _, _ = qkv(S, seed=14, device="cpu", past=past)
+    import ctypes
+    import os
+    from cuda_inf_amd._lib import call
+    kd, vd = k0.to(dev), v0.to(dev)
+    call("cia_layer_append", ctypes.byref(L._s), kd.data_ptr(), vd.data_ptr(), past + S, 0,
+         torch.cuda.current_stream().cuda_stream)
+    ref.append(_u16(k0), _u16(v0), 0)
+    qd, out = q.to(dev), torch.empty((S, 32, 64), dtype=torch.float16, device=dev)
+    args = (qd, L.kc8, L.vc8, L.ksc, L.vsc, L.ktail, L.vtail, L.committed, out, None, S, past, 0.125)
+    K.attention_fused(*args)
+    torch.cuda.synchronize()
+    nth = max(1, min(16, os.cpu_count() or 1))
+    _, r32 = orc.attention_fused_mt(_u16(q), ref, S, past, nthreads=nth)
+    assert_close_f16(_u16(out), r32)
+    if past >= 64:  # the same queries 64 positions earlier: later keys are masked
+        K.attention_fused(*args[:11], past - 64, 0.125)
+        torch.cuda.synchronize()
+        _, r32 = orc.attention_fused_mt(_u16(q), ref, S, past - 64, nthreads=nth)
+        assert_close_f16(_u16(out), r32)
+
+
 def test_decode_steps_through_commit(orc, cia, dev):
     """Decode steps that cross a group boundary (tail fills, commit, new tail)."""
     from cuda_inf_amd.layer import AttnLayer
