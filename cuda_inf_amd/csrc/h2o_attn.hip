@@ -24,7 +24,8 @@
 // Every product, sum and fma above is a single IEEE-rounded operation;
 // contraction is off in this file so the compiler adds no fusions.
 //
-// Two launches per chunk of up to kChunk queries, each spread over the
+// From kManyMin queries on, k_h2o_stats, k_h2o_weights and k_h2o_chain below.
+// Fewer: two launches per chunk of up to kChunk queries, each spread over the
 // whole chip (the reference's one block of 32 threads per query scans the
 // buffer serially):
 //   k_h2o_scores  (64-slot block, kv head, query): one wave per query head
@@ -119,6 +120,8 @@ __device__ __forceinline__ int wave_id() {
 }
 
 typedef int i32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) void lds_void_t;
+typedef __attribute__((address_space(1))) void gbl_void_t;
 typedef __attribute__((address_space(3))) i32x2 lds_i32x2_t;
 
 // piece swizzle of V row r in LDS (4 pieces of 16 bytes per 64-byte row): a
@@ -557,6 +560,335 @@ __global__ __launch_bounds__(1024) void k_h2o_mass(H2oArgs a, int nsw) {
   }
 }
 
+// ---------------------------------------------------------------- many queries
+// A prompt's attention mass.  attn_sum[t] takes one rounded add per (query,
+// head) in order, so 1024 queries are 32768 dependent adds a slot (about 60 us)
+// whatever else is done; the rest -- 64 fused multiply-adds and an exponential
+// per (query, head, slot), twice, since the weights need every block's maximum
+// first -- has to run beside that chain and on the whole chip.  Three launches
+// for any number of queries (the outputs come from the matrix cores, in a
+// launch of their own, prefill_split.hip):
+//   k_h2o_stats    m_b and l_b: a wave holds a block's 64 keys of one kv head
+//                  in registers, lane = slot, for kStQ queries; q comes from
+//                  LDS by broadcast and enters the fma as fp16.
+//   k_h2o_weights  w_b in place of l_b, lane = (query, head) row.
+//   k_h2o_chain    a workgroup per kSl slots: eight waves, one per kv head,
+//                  take s again and the products p = exp_det(s - m_b) w_b, lane
+//                  = (slot, query, head) with the slot's key in registers; a
+//                  ninth adds the previous step's products to the masses.  The
+//                  products never leave LDS: storing e for every slot instead
+//                  bounds the queries in flight by the scratch, 16 at a time.
+// Queries that see no slot of a block or workgroup are passed over; a product
+// of a slot that its query does not see is -0, which leaves any sum as it is.
+// (S = 1024 into an empty 2048-slot buffer: per 16 queries a scores and a mass
+// launch, its chain on one workgroup per 256 slots, 2500 us in all; as here 300:
+// stats 81, weights 7, chain 179, outputs 28.)
+struct MassArgs {
+  const uint16_t* q;  // first query row of the chunk
+  const uint8_t* kf;
+  const uint16_t* ks;
+  const int32_t* slot_pos;
+  float* attn_sum;
+  f32x2* ml;  // [nblk][nq * 32]: m_b, then l_b or w_b
+  int n_live, nblk, nq, qpos0;
+  float scale;
+};
+// Queries from which these launches run instead of the pair per 16 queries: few
+// queries leave the chip idle in four launches where the pair is two.  (Pair /
+// these, us, attention over 2048 slots: S = 8 28 / 37, 16 50 / 41, 64 191 /
+// 68; a prompt into an empty buffer, with placement: 8 29 / 30, 16 47 / 36,
+// 64 136 / 37.)
+constexpr int kManyMin = 16;
+constexpr int kStQ = 4;  // queries of a stats group
+
+// 16-byte piece swizzle of K row r in a wave's LDS: each lane then reads one
+// whole row, and lanes r, r + 4, .. of a bank window take distinct pieces
+__device__ __forceinline__ int ksw(int r) { return (r >> 2) & 3; }
+
+// a key row as k(t)[d] = e4m3(byte d) * scale
+__device__ __forceinline__ void key_row(const u32x4 (&w)[4], float ksc, float (&k)[D]) {
+#pragma unroll
+  for (int p = 0; p < 4; p++)
+#pragma unroll
+    for (int x = 0; x < 4; x++) {
+      const f32x2 lo = e4m3x2_to_f32<false>(w[p][x]), hi = e4m3x2_to_f32<true>(w[p][x]);
+      k[16 * p + 4 * x + 0] = lo[0] * ksc;
+      k[16 * p + 4 * x + 1] = lo[1] * ksc;
+      k[16 * p + 4 * x + 2] = hi[0] * ksc;
+      k[16 * p + 4 * x + 3] = hi[1] * ksc;
+    }
+}
+
+// grid = (2 nblk, ceil(nq / (kStQ ngrp))), block = 256: wave w, kv head 4
+// (blockIdx.x & 1) + w, ngrp groups of kStQ queries
+__global__ __launch_bounds__(256) void k_h2o_stats(MassArgs a, int ngrp) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[4][64 * D + kStQ * GQA * D * 2];
+  const int wv = wave_id(), lane = threadIdx.x & 63;
+  // (the block rotates with the query group: workgroups go to the XCDs by their
+  // number, and in a prompt the first blocks are seen by the most queries)
+  const int blk = ((blockIdx.x >> 1) + blockIdx.y) % a.nblk, g = 4 * (blockIdx.x & 1) + wv;
+  const int ib = blockIdx.y * kStQ * ngrp, ie = min(ib + kStQ * ngrp, a.nq);
+  uint8_t* kl = lds[wv];
+  uint16_t* ql = (uint16_t*)(kl + 64 * D);
+  const int t0 = blk * 64, t = t0 + lane;
+  const bool live = t < a.n_live;
+  const int tc = live ? t : a.n_live - 1;
+  const int sp = live ? a.slot_pos[tc] : 0x7FFFFFFF;
+  const uint16_t ks16 = a.ks[(size_t)tc * NKV + g];
+  // the block's K rows, 4 neighbouring lanes to a row (rows past the last
+  // slot read it again), through LDS to one row a lane; q beside them (32
+  // lanes to a query's 4 heads), a group ahead
+  u32x4 kr[4], qr[kStQ / 2];
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const int r = min(t0 + 16 * j + (lane >> 2), a.n_live - 1);
+    kr[j] = *(const u32x4*)(a.kf + ((size_t)r * NKV + g) * D + 16 * (lane & 3));
+  }
+  auto load_q = [&](int i0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < kStQ / 2; j++)
+      qr[j] = *(const u32x4*)(a.q + ((size_t)min(i0 + 2 * j + (lane >> 5), a.nq - 1) * NH + g * GQA) * D + 8 * (lane & 31));
+  };
+  load_q(ib);
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const int r = 16 * j + (lane >> 2);
+    *(u32x4*)(kl + r * 64 + 16 * ((lane & 3) ^ ksw(r))) = kr[j];
+  }
+  u32x4 w[4];
+#pragma unroll
+  for (int p = 0; p < 4; p++) w[p] = *(const u32x4*)(kl + lane * 64 + 16 * (p ^ ksw(lane)));
+  float k[D];
+  key_row(w, h2f(ks16), k);
+#pragma unroll 1
+  for (int i = ib; i < ie; i++) {
+    const int r = (i - ib) % kStQ;
+    if (r == 0) {
+#pragma unroll
+      for (int j = 0; j < kStQ / 2; j++) *(u32x4*)(ql + 512 * j + 8 * lane) = qr[j];
+      if (i + kStQ < ie) load_q(i + kStQ);
+    }
+    f32x2* ml = a.ml + (size_t)blk * (a.nq * NH) + i * NH + g * GQA;
+    const bool ok = sp <= a.qpos0 + i;
+    if (!__any(ok)) {
+      if (lane < GQA) ml[lane] = f32x2{kNegInf, 0.0f};
+      continue;
+    }
+    // (two heads at a time: their q rows are what the registers hold beside k)
+#pragma unroll 1
+    for (int h0 = 0; h0 < GQA; h0 += 2) {
+      const uint16_t* q = ql + (r * GQA + h0) * D;
+      float s[2] = {0.0f, 0.0f};
+#pragma unroll
+      for (int d = 0; d < D; d += 8)
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          const u32x4 qq = *(const u32x4*)(q + h * D + d);
+#pragma unroll
+          for (int x = 0; x < 4; x++) {
+            s[h] = __builtin_fmaf(h2f((uint16_t)qq[x]), k[d + 2 * x], s[h]);
+            s[h] = __builtin_fmaf(h2f((uint16_t)(qq[x] >> 16)), k[d + 2 * x + 1], s[h]);
+          }
+        }
+      f32x2 o[2];
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        s[h] = ok ? s[h] * a.scale : kNegInf;
+        const float mb = wave_max_fast(s[h]);
+        o[h] = f32x2{mb, wave_tree_sum(ok ? exp_det(s[h] - mb) : 0.0f)};
+      }
+      if (lane < 2) ml[h0 + lane] = lane == 0 ? o[0] : o[1];
+    }
+  }
+}
+
+// grid = ceil(nq * 32 / 64), block = 64
+constexpr int kWtB = 16;  // blocks of a row read together
+__global__ __launch_bounds__(64) void k_h2o_weights(MassArgs a) {
+  const int nrow = a.nq * NH, row = blockIdx.x * 64 + threadIdx.x;  // (whole waves: 32 | nrow)
+  f32x2* ml = a.ml + min(row, nrow - 1);
+  f32x2 u[kWtB];
+  auto load = [&](int c0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < kWtB; k++) u[k] = ml[(size_t)min(c0 + k, a.nblk - 1) * nrow];
+  };
+  float m = kNegInf;
+  for (int c0 = 0; c0 < a.nblk; c0 += kWtB) {
+    load(c0);
+#pragma unroll
+    for (int k = 0; k < kWtB; k++) m = __builtin_fmaxf(m, u[k][0]);  // (a repeat changes nothing)
+  }
+  float l = 0.0f;
+  for (int c0 = 0; c0 < a.nblk; c0 += kWtB) {  // in block order
+    if (a.nblk > kWtB) load(c0);
+#pragma unroll
+    for (int k = 0; k < kWtB; k++) {
+      if (c0 + k < a.nblk) l = l + u[k][1] * (u[k][0] == kNegInf ? 0.0f : exp_det(u[k][0] - m));
+    }
+  }
+  const float inv = 1.0f / l;
+  for (int c0 = 0; c0 < a.nblk; c0 += kWtB) {
+    if (a.nblk > kWtB) load(c0);
+#pragma unroll
+    for (int k = 0; k < kWtB; k++)
+      if (c0 + k < a.nblk && row < nrow)
+        ml[(size_t)(c0 + k) * nrow][1] = (u[k][0] == kNegInf ? 0.0f : exp_det(u[k][0] - m)) * inv;
+  }
+}
+
+// grid = ceil(n_live / kSl), block = 576.  A step is kR queries.
+template <int kSl>
+__global__ __launch_bounds__(64 * (NKV + 1)) void k_h2o_chain(MassArgs a) {
+  constexpr int kR = 16 / kSl;  // queries of a step
+  constexpr int kQB = kR * GQA * D * 2;  // bytes of a wave's q rows
+  // one object (with two, the compiler makes every LDS read wait for the DMA in
+  // flight): the waves' q rows, twice [NKV][kQB], then the products, twice
+  // f32x4 [query][kv head][slot] of 4 heads
+  __shared__ __attribute__((aligned(16))) uint8_t lds[2 * NKV * kQB + 2 * kR * NKV * kSl * 16];
+  auto prod = [&](int n, int r, int g, int s) {
+    return (f32x4*)(lds + 2 * NKV * kQB) + (((n & 1) * kR + r) * NKV + g) * kSl + s;
+  };
+  const int wv = wave_id(), lane = threadIdx.x & 63;
+  const int t0 = blockIdx.x * kSl, t = t0 + lane % kSl, tc = min(t, a.n_live - 1);
+  const int sp = t < a.n_live ? a.slot_pos[tc] : 0x7FFFFFFF;
+  // the first query that sees a slot of the workgroup
+  int lo = sp;
+#pragma unroll
+  for (int o = 1; o < kSl; o <<= 1) lo = min(lo, __shfl_xor(lo, o));
+  lo = __builtin_amdgcn_readfirstlane(lo);
+  const int first = lo <= a.qpos0 ? 0 : (lo - a.qpos0 < a.nq ? (lo - a.qpos0) / kR : (a.nq + kR - 1) / kR);
+  const int nstep = (a.nq + kR - 1) / kR;
+  // a step's barrier: LDS only (__syncthreads would wait for the next step's
+  // loads as well)
+  auto step_barrier = [&]() __attribute__((always_inline)) {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  if (wv == NKV) {
+    // ---- the chain: lane = slot, one step behind
+    float acc = a.attn_sum[tc];
+    for (int n = first; n <= nstep; n++) {
+      if (n > first) {
+        // (a query's products requested while the one before is added)
+        const f32x4* p = prod(n - 1, 0, 0, lane % kSl);
+        f32x4 v[2][NKV];
+#pragma unroll
+        for (int g = 0; g < NKV; g++) v[0][g] = p[g * kSl];
+#pragma unroll
+        for (int r = 0; r < kR; r++) {
+          if (r + 1 < kR)
+#pragma unroll
+            for (int g = 0; g < NKV; g++) v[(r + 1) & 1][g] = p[((r + 1) * NKV + g) * kSl];
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int g = 0; g < NKV; g++)
+#pragma unroll
+            for (int h = 0; h < GQA; h++) acc = acc + v[r & 1][g][h];
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      step_barrier();
+    }
+    if (lane < kSl && t < a.n_live) a.attn_sum[t] = acc;
+    return;
+  }
+  // ---- products of kv head g
+  const int g = wv, j = lane / kSl, r = j >> 2, h = j & 3;
+  const uint8_t* kp = a.kf + ((size_t)tc * NKV + g) * D;
+  u32x4 w[4];
+#pragma unroll
+  for (int p = 0; p < 4; p++) w[p] = *(const u32x4*)(kp + 16 * p);
+  const float ksc = h2f(a.ks[(size_t)tc * NKV + g]);
+  // a step's q rows by DMA into LDS (16-byte pieces lane, lane + 64, ..; row
+  // (query, head)'s piece p lies at p ^ (row & 7)) and (m_b, w_b), one step ahead
+  constexpr int kPc = kQB / 16;  // pieces: 32 a query
+  constexpr int kLd = (kPc + 63) / 64;
+  // (buffer loads: one lane offset for every step, rows past the chunk read 0)
+  const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)a.q, 0, a.nq * (NH * D * 2), 0x00020000);
+  const int row0 = lane / 8;  // of piece `lane`; piece lane + 64 c: row0 + 8 c, two queries on
+  const int qo = ((row0 >> 2) * NH + g * GQA + (row0 & 3)) * (D * 2) + 16 * ((lane & 7) ^ row0);
+  const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(a.ml + (size_t)(t0 >> 6) * (a.nq * NH)), 0, a.nq * (NH * 8), 0x00020000);
+  const int mo = (r * NH + g * GQA + h) * 8;
+  auto fetch = [&](int n, f32x2& mw) __attribute__((always_inline)) {
+    mw = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rm, mo, n * kR * (NH * 8), 0));
+#pragma unroll
+    for (int c = 0; c < kLd; c++)
+      if (kPc >= 64 || lane < kPc)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (lds_void_t*)(lds + ((n & 1) * NKV + g) * kQB + 1024 * c), 16, qo,
+                                                 (n * kR + 2 * c) * (NH * D * 2), 0, 0);
+  };
+  // (two steps' (m_b, w_b) in registers of their own: a copy from one to the
+  // other would wait for the load)
+  f32x2 mw0, mw1;
+  if (first < nstep) fetch(first, mw0);
+  float k[D];
+  key_row(w, ksc, k);
+  auto step = [&](int n, f32x2& cur, f32x2& next) __attribute__((always_inline)) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this step's q rows
+    asm volatile("" ::: "memory");         // (no LDS read moves above the wait)
+    if (n + 1 < nstep) fetch(n + 1, next);
+    const uint8_t* qw = lds + ((n & 1) * NKV + g) * kQB;
+    float s = 0.0f;
+#pragma unroll
+    for (int p = 0; p < 8; p++) {
+      const u32x4 qq = *(const u32x4*)(qw + j * 128 + 16 * (p ^ (j & 7)));
+#pragma unroll
+      for (int x = 0; x < 4; x++) {
+        s = __builtin_fmaf(h2f((uint16_t)qq[x]), k[8 * p + 2 * x], s);
+        s = __builtin_fmaf(h2f((uint16_t)(qq[x] >> 16)), k[8 * p + 2 * x + 1], s);
+      }
+      if (p & 1) __builtin_amdgcn_sched_barrier(0);  // (few of q's pieces in registers at once)
+    }
+    const int i = n * kR + r;
+    const float p = exp_det(s * a.scale - cur[0]) * cur[1];
+    ((float*)prod(n, r, g, lane % kSl))[h] = i < a.nq && sp <= a.qpos0 + i ? p : -0.0f;
+    step_barrier();
+  };
+  for (int n = first; n < nstep; n += 2) {
+    step(n, mw0, mw1);
+    if (n + 1 < nstep) step(n + 1, mw1, mw0);
+  }
+  step_barrier();
+}
+
+// attn_sum of S queries over the live slots.  ws: 64 floats per (query, block)
+// of a chunk, the chunk being what ws_bytes holds (h2o_ws_bytes(S, n_live):
+// all S queries up to 1048).
+static int h2o_mass_many(const uint16_t* q, const uint8_t* kf, const uint16_t* ks,
+                         const int32_t* slot_pos, int n_live, float* attn_sum, int S, int past,
+                         float scale, void* ws, int64_t ws_bytes, hipStream_t s) {
+  MassArgs a{nullptr, kf, ks, slot_pos, attn_sum, (f32x2*)ws, n_live, (n_live + 63) / 64, 0, 0, scale};
+  const int64_t fit = ws_bytes / ((int64_t)NH * a.nblk * (int64_t)sizeof(f32x2));
+  if (fit < 1) return CIA_ERR_ARG;
+  const int Q = (int)std::min<int64_t>(std::min<int64_t>(S, fit), 65536);  // (32-bit offsets)
+  for (int c0 = 0; c0 < S; c0 += Q) {
+    a.q = q + (size_t)c0 * NH * D;
+    a.nq = std::min(Q, S - c0);
+    a.qpos0 = past + c0;
+    // (about 8 workgroups per compute unit: each pays for its keys once)
+    const int grp = (a.nq + kStQ - 1) / kStQ, ngrp = std::max(1, std::min(16, grp * 2 * a.nblk / 4096));
+    hipLaunchKernelGGL(k_h2o_stats, dim3(2 * a.nblk, (grp + ngrp - 1) / ngrp), dim3(256), 0, s, a, ngrp);
+    int st = launch_status();
+    if (st) return st;
+    hipLaunchKernelGGL(k_h2o_weights, dim3((a.nq * NH + 63) / 64), dim3(64), 0, s, a);
+    if ((st = launch_status())) return st;
+    // the fewest slots a workgroup that leave at most one per compute unit
+    const dim3 block(64 * (NKV + 1));
+    if (n_live <= 4 * 256)
+      hipLaunchKernelGGL(k_h2o_chain<4>, dim3((n_live + 3) / 4), block, 0, s, a);
+    else if (n_live <= 8 * 256)
+      hipLaunchKernelGGL(k_h2o_chain<8>, dim3((n_live + 7) / 8), block, 0, s, a);
+    else
+      hipLaunchKernelGGL(k_h2o_chain<16>, dim3((n_live + 15) / 16), block, 0, s, a);
+    if ((st = launch_status())) return st;
+  }
+  return CIA_OK;
+}
+
 // the placement keys' region after the partials (16-byte aligned)
 int64_t h2o_keys_offset(int S, int C) {
   const int64_t sq = std::min(S, kChunk), nblk = (C + 63) / 64;
@@ -571,6 +903,11 @@ int64_t h2o_ws_bytes(int S, int C) {
 }  // namespace cia
 
 using namespace cia;
+
+extern "C" __attribute__((visibility("hidden"))) int cia_h2o_out(
+    const uint16_t* q, const uint8_t* kf, const uint8_t* vf, const uint16_t* ks,
+    const uint16_t* vs, const int32_t* slot_pos, int n_live, uint16_t* out, int S, int past,
+    float scale, void* stream);
 
 extern "C" int64_t cia_h2o_workspace_bytes(int S, int C) {
   return (S < 0 || C < 0) ? 0 : h2o_ws_bytes(S, C);
@@ -591,6 +928,12 @@ extern "C" int cia_attention_h2o(const uint16_t* q, const uint8_t* kf, const uin
               CIA_ERR_ALIGN);
   hipStream_t s = (hipStream_t)stream;
   const int nblk = (n_live + 63) / 64;
+  // (8-byte output stores, 32-bit slot offsets)
+  if (S >= kManyMin && aligned(out, 8) && n_live <= (1 << 22)) {
+    const int st = cia_h2o_out(q, kf, vf, ks, vs, slot_pos, n_live, out, S, past, scale, stream);
+    if (st) return st;
+    return h2o_mass_many(q, kf, ks, slot_pos, n_live, attn_sum, S, past, scale, ws, ws_bytes, s);
+  }
   for (int c0 = 0; c0 < S; c0 += kChunk) {
     const int sq = std::min(kChunk, S - c0);
     H2oArgs a;

@@ -29,6 +29,7 @@
 namespace cia {
 
 typedef int i32x2 __attribute__((ext_vector_type(2)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) i32x2 lds_i32x2_t;
 
 // 16-byte piece swizzle of LDS row r (4 pieces of 64 bytes): bits 2, 3, 4 of
@@ -39,17 +40,27 @@ __device__ __forceinline__ int ps_sw(int r) {
   return (((r >> 2) ^ (r >> 4)) & 1) | (((r >> 2) ^ (r >> 3)) & 2);
 }
 
+// What differs over the H2O slot buffer (attention_h2o's outputs,
+// engine.cu:337-384): tiles of 64 slots, a scale per slot, and the mask from
+// slot_pos.  The tile's slots' scales and positions pass through the wave's
+// LDS; a K scale multiplies its fp32 scores, a V scale its fp16 row.
+struct SlotArgs {
+  const int32_t* slot_pos;
+  int n_live;
+};
+
 constexpr int kPsORow = 68;  // floats between two queries of a wave's partial O
-// bytes of a wave's LDS: the K and V tiles; then m, l and O per query
-constexpr int ps_wave_bytes(int qt) {
-  const int merge = 16 * qt * (kPsORow + 2) * 4;
-  return merge > 8192 ? merge : 8192;
+// bytes of a wave's LDS: the K and V tiles (and 64 slots' K scales, positions
+// and V scales); then m, l and O per query
+constexpr int ps_wave_bytes(bool slots, int qt) {
+  const int merge = 16 * qt * (kPsORow + 2) * 4, tiles = 8192 + (slots ? 64 * 10 : 0);
+  return merge > tiles ? merge : tiles;
 }
 
 // grid = 8 kv heads * 4 * nq (nq = ceil(S / (16 kQT))), block = 64 kW
-template <int kQT, int kW>
-__global__ __launch_bounds__(64 * kW) void k_prefill_split(PrefillArgs a) {
-  constexpr int kWB = ps_wave_bytes(kQT);
+template <bool kSlots, int kQT, int kW>
+__global__ __launch_bounds__(64 * kW) void k_prefill_split(PrefillArgs a, SlotArgs sl) {
+  constexpr int kWB = ps_wave_bytes(kSlots, kQT);
   __shared__ __attribute__((aligned(16))) uint8_t lds[kW * kWB];
   const int tid = threadIdx.x, l = tid & 63, n = l & 15, b = l >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -58,17 +69,37 @@ __global__ __launch_bounds__(64 * kW) void k_prefill_split(PrefillArgs a) {
   const int g = blockIdx.x & 7, h = g * GQA + ((blockIdx.x >> 3) & 3);
   const int q0 = (a.nblk - 1 - (int)(blockIdx.x >> 5)) * 16 * kQT;
   const int qmin = a.past + q0, qlast = a.past + min(q0 + 16 * kQT - 1, a.S - 1);
-  const int ntile = (qlast >> 6) + 1, nfp8 = a.committed >> 6;
+  const int ntile = kSlots ? (sl.n_live + 63) >> 6 : (qlast >> 6) + 1;
+  const int nfp8 = kSlots ? ntile : a.committed >> 6;
   uint8_t* kt = lds + w * kWB;
   uint8_t* vt = kt + 4096;
+  float* lks = (float*)(kt + 8192);
+  int* lpos = (int*)(kt + 8192 + 256);
+  _Float16* lvs = (_Float16*)(kt + 8192 + 512);
 
   struct Tile {
     u32x4 k[4], v[4];
-    uint16_t ks, vs;
+    uint16_t ks, vs;  // the group's; kSlots: those of slot l of the tile
+    int pos;
   };
   // (uniform bases and one 32-bit lane offset)
   const uint32_t loff = (uint32_t)((l >> 2) * (NKV * D) + 16 * (l & 3));
   auto load = [&](int j, Tile& t) __attribute__((always_inline)) {
+    if constexpr (kSlots) {
+      // (slots past the last read it again, at a position no query sees)
+      const int r0 = 64 * j, last = sl.n_live - 1;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const uint32_t o = (uint32_t)(min(r0 + 16 * i + (l >> 2), last) * (NKV * D) + 16 * (l & 3));
+        t.k[i] = *(const u32x4*)(a.kc8 + g * D + o);
+        t.v[i] = *(const u32x4*)(a.vc8 + g * D + o);
+      }
+      const int r = min(r0 + l, last);
+      t.ks = a.ksc[r * NKV + g];
+      t.vs = a.vsc[r * NKV + g];
+      t.pos = r0 + l <= last ? sl.slot_pos[r] : 0x7fffffff;
+      return;
+    }
     const size_t o = (size_t)j * (G * NKV * D) + g * D;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -128,7 +159,18 @@ __global__ __launch_bounds__(64 * kW) void k_prefill_split(PrefillArgs a) {
       }
     }
     // (masked scores become -inf in place: c > 0 keeps them there)
-    if (64 * j + 63 > qmin) {
+    if constexpr (kSlots) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const f32x4 ks = *(const f32x4*)(lks + 16 * k + 4 * b);
+        const i32x4 pos = *(const i32x4*)(lpos + 16 * k + 4 * b);
+#pragma unroll
+        for (int t = 0; t < kQT; t++)
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            S[t][k][i] = pos[i] > qmin + 16 * t + n ? -__builtin_inff() : S[t][k][i] * ks[i];
+      }
+    } else if (64 * j + 63 > qmin) {
 #pragma unroll
       for (int t = 0; t < kQT; t++)
 #pragma unroll
@@ -150,20 +192,37 @@ __global__ __launch_bounds__(64 * kW) void k_prefill_split(PrefillArgs a) {
   int first = 1;
   asm("" : "+s"(first));  // (opaque: the loop's first pass is not peeled into code of its own)
   for (int j = w; j < nf; j += kW) {
-    const float c = __builtin_fmaxf(h2f((uint16_t)pf_late(cur.ks)) * a.qscale, 1e-30f);
-    const float vs = h2f((uint16_t)pf_late(cur.vs));
+    float c = 1.0f, vs = 1.0f;
+    bool seen = true;  // by some query of the workgroup
+    if constexpr (kSlots) {
+      seen = __any(cur.pos <= qlast);
+      lks[l] = h2f(cur.ks) * a.qscale;
+      lpos[l] = cur.pos;
+      lvs[l] = __builtin_bit_cast(_Float16, cur.vs);
+    } else {
+      c = __builtin_fmaxf(h2f((uint16_t)pf_late(cur.ks)) * a.qscale, 1e-30f);
+      vs = h2f((uint16_t)pf_late(cur.vs));
+    }
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       *(u32x4*)(kt + (i & 1 ? wo1 : wo0) + 1024 * i) = cur.k[i];
       *(u32x4*)(vt + (i & 1 ? wo1 : wo0) + 1024 * i) = cur.v[i];
     }
     if (j + kW < nf) load(j + kW, cur);
+    if (!seen) continue;
     auto kop = [&](int k, f16x8& k0, f16x8& k1) __attribute__((always_inline)) {
       const u32x4 kk = *(const u32x4*)(kt + (k & 1 ? ko1 : ko0) + 1024 * k);
       k0 = pf_cvt8(kk[0], kk[1]);
       k1 = pf_cvt8(kk[2], kk[3]);
     };
     auto pv = [&](const f16x8 (&P)[kQT][2]) __attribute__((always_inline)) {
+      f16x8 sc[2];
+      if constexpr (kSlots)
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+          const f16x4 lo = *(const f16x4*)(lvs + 32 * u + 4 * b), hi = *(const f16x4*)(lvs + 32 * u + 16 + 4 * b);
+          sc[u] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
 #pragma unroll
       for (int d = 0; d < 4; d++) {
         f16x8 vop[2];
@@ -172,9 +231,15 @@ __global__ __launch_bounds__(64 * kW) void k_prefill_split(PrefillArgs a) {
           const i32x2 raw = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
               (lds_i32x2_t*)(vt + (vo ^ 16 * d) + 2048 * u));
           vop[u] = pf_cvt8((uint32_t)raw[0], (uint32_t)raw[1]);
+          if constexpr (kSlots) vop[u] *= sc[u];
         }
 #pragma unroll
         for (int t = 0; t < kQT; t++) {
+          if constexpr (kSlots) {
+            O[t][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vop[0], P[t][0], O[t][d], 0, 0, 0);
+            O[t][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vop[1], P[t][1], O[t][d], 0, 0, 0);
+            continue;
+          }
           f32x4 T = __builtin_amdgcn_mfma_f32_16x16x32_f16(vop[0], P[t][0], zero, 0, 0, 0);
           T = __builtin_amdgcn_mfma_f32_16x16x32_f16(vop[1], P[t][1], T, 0, 0, 0);
 #pragma unroll
@@ -185,7 +250,7 @@ __global__ __launch_bounds__(64 * kW) void k_prefill_split(PrefillArgs a) {
     attend(j, c, first != 0, kop, pv);
     first = 0;
   }
-  if (ntile > nfp8 && nfp8 % kW == w) {
+  if (!kSlots && ntile > nfp8 && nfp8 % kW == w) {
     // the fp16 tail: K straight into operand order, V rows through the wave's
     // LDS (rows past the last token are zero), read back one value at a time
     const int nvalid = a.past + a.S - a.committed;
@@ -268,11 +333,31 @@ using namespace cia;
 
 namespace {
 
-template <int kQT, int kW>
-int split_launch(PrefillArgs a, hipStream_t s) {
+template <bool kSlots, int kQT, int kW>
+int split_launch(PrefillArgs a, const SlotArgs& sl, hipStream_t s) {
   a.nblk = (a.S + 16 * kQT - 1) / (16 * kQT);
-  hipLaunchKernelGGL((k_prefill_split<kQT, kW>), dim3(8 * GQA * a.nblk), dim3(64 * kW), 0, s, a);
+  hipLaunchKernelGGL((k_prefill_split<kSlots, kQT, kW>), dim3(8 * GQA * a.nblk), dim3(64 * kW), 0, s,
+                     a, sl);
   return launch_status();
+}
+
+// Shape: one 16-query tile per wave while those units fit the chip at once
+// (the more waves on the keys, the more keys there are), or while there are
+// few keys; then two, so that a K / V tile's conversions serve 32 queries.
+// (1 x 4, 1 x 8, 1 x 16, 2 x 4, 2 x 8 waves, us: 77 at 0 4.8 5.2 5.5 5.5 5.5;
+// 77 at 1000 8.7 7.9 7.2 11.6 8.9; 77 at 9000 33 27 25 51 34; 1000 at 0 16.8
+// 20.9 32 18.5 22.4; 1500 at 0 29.5 34 53 28.9 36; 200 at 4000 25 25 27 28 20;
+// 1000 at 8000 175 167 180 131 125.)
+template <bool kSlots>
+int split_shape(const PrefillArgs& a, const SlotArgs& sl, int tiles, hipStream_t st) {
+  if (NH * ((a.S + 15) / 16) <= 256) {
+    if (tiles <= 8) return split_launch<kSlots, 1, 4>(a, sl, st);
+    if (tiles <= 12) return split_launch<kSlots, 1, 8>(a, sl, st);
+    return split_launch<kSlots, 1, 16>(a, sl, st);
+  }
+  if (tiles <= 20) return split_launch<kSlots, 1, 4>(a, sl, st);
+  if (tiles <= 40) return split_launch<kSlots, 2, 4>(a, sl, st);
+  return split_launch<kSlots, 2, 8>(a, sl, st);
 }
 
 }  // namespace
@@ -292,27 +377,21 @@ extern "C" __attribute__((visibility("hidden"))) int cia_prefill_split_wins(int 
   return split < block;
 }
 
-// Shape: one 16-query tile per wave while those units fit the chip at once
-// (the more waves on the keys, the more keys there are), or while there are
-// few keys; then two, so that a K / V tile's conversions serve 32 queries.
-// (1 x 4, 1 x 8, 1 x 16, 2 x 4, 2 x 8 waves, us: 77 at 0 4.8 5.2 5.5 5.5 5.5;
-// 77 at 1000 8.7 7.9 7.2 11.6 8.9; 77 at 9000 33 27 25 51 34; 1000 at 0 16.8
-// 20.9 32 18.5 22.4; 1500 at 0 29.5 34 53 28.9 36; 200 at 4000 25 25 27 28 20;
-// 1000 at 8000 175 167 180 131 125.)
 extern "C" __attribute__((visibility("hidden"))) int cia_prefill_split(
     const uint16_t* q, const uint8_t* kc8, const uint8_t* vc8, const uint16_t* ksc,
     const uint16_t* vsc, const uint16_t* ktail, const uint16_t* vtail, int committed,
     uint16_t* out, int S, int past, float scale, void* stream) {
   const PrefillArgs a{q, kc8, vc8, ksc, vsc, ktail, vtail, committed, out, S, past,
                       scale * kPfLog2e, 0};
-  hipStream_t st = (hipStream_t)stream;
-  const int tiles = (past + S + 63) / 64;
-  if (NH * ((S + 15) / 16) <= 256) {
-    if (tiles <= 8) return split_launch<1, 4>(a, st);
-    if (tiles <= 12) return split_launch<1, 8>(a, st);
-    return split_launch<1, 16>(a, st);
-  }
-  if (tiles <= 20) return split_launch<1, 4>(a, st);
-  if (tiles <= 40) return split_launch<2, 4>(a, st);
-  return split_launch<2, 8>(a, st);
+  return split_shape<false>(a, SlotArgs{}, (past + S + 63) / 64, (hipStream_t)stream);
+}
+
+// attention_h2o's outputs for S queries over n_live slots (arguments checked
+// by cia_attention_h2o)
+extern "C" __attribute__((visibility("hidden"))) int cia_h2o_out(
+    const uint16_t* q, const uint8_t* kf, const uint8_t* vf, const uint16_t* ks,
+    const uint16_t* vs, const int32_t* slot_pos, int n_live, uint16_t* out, int S, int past,
+    float scale, void* stream) {
+  const PrefillArgs a{q, kf, vf, ks, vs, nullptr, nullptr, 0, out, S, past, scale * kPfLog2e, 0};
+  return split_shape<true>(a, SlotArgs{slot_pos, n_live}, (n_live + 63) / 64, (hipStream_t)stream);
 }

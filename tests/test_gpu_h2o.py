@@ -318,3 +318,13 @@ def test_h2o_layers_sharing_ws_mass(cia, dev):
         for name in ("hattn", "d_slotpos", "kf", "vf", "ks", "vs"):
             x, y = getattr(la[l], name), getattr(lb[l], name)
             assert torch.equal(x.view(torch.uint8), y.view(torch.uint8)), (l, name)
+
+
+@pytest.mark.parametrize("n_live,S,past,seed", [
+    (3, 16, 0, 40), (64, 33, 10, 41), (1030, 17, 900, 42), (2500, 16, 3000, 43),
+    (70, 1100, 30, 44), (1024, 15, 600, 45), (257, 130, 200, 46)])
+def test_attention_h2o_many_queries(orc, cia, dev, n_live, S, past, seed):
+    """The many-query launches: each slots-per-workgroup choice, slots that end
+    inside a workgroup and a block, queries that end inside a step, more
+    queries than the scratch holds at once (1048), the last S of the pair."""
+    test_attention_h2o_kernel(orc, cia, dev, n_live, S, past, seed)
