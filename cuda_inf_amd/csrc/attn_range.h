@@ -22,12 +22,18 @@ struct Group64Cache {
   const uint16_t* ktail;
   const uint16_t* vtail;
   int committed;
+  // the token at position fresh is not in the tail yet but at knew, vnew
+  // [8][64] (fresh = -1: none)
+  const uint16_t* knew;
+  const uint16_t* vnew;
+  int fresh;
 };
 
 // 16 dequantised values of key/value row t (kv head kvh), dims d0..d0+15
 __device__ __forceinline__ void load_row16(const uint8_t* c8, const uint16_t* sc,
-                                           const uint16_t* tail, int committed, int t,
-                                           int kvh, int d0, float* x) {
+                                           const uint16_t* tail, const uint16_t* fresh_row,
+                                           int fresh, int committed, int t, int kvh, int d0,
+                                           float* x) {
   if (t < committed) {
     const u32x4 b = *(const u32x4*)(c8 + ((size_t)t * NKV + kvh) * D + d0);
     const float s = h2f(sc[(t / G) * NKV + kvh]);
@@ -40,7 +46,7 @@ __device__ __forceinline__ void load_row16(const uint8_t* c8, const uint16_t* sc
       x[4 * w + 3] = hi[1] * s;
     }
   } else {
-    const uint16_t* p = tail + ((size_t)(t - committed) * NKV + kvh) * D + d0;
+    const uint16_t* p = (t == fresh ? fresh_row : tail + (size_t)(t - committed) * NKV * D) + kvh * D + d0;
     const u32x4 a = *(const u32x4*)p, b = *(const u32x4*)(p + 8);
 #pragma unroll
     for (int w = 0; w < 4; w++) {
@@ -50,6 +56,12 @@ __device__ __forceinline__ void load_row16(const uint8_t* c8, const uint16_t* sc
       x[8 + 2 * w + 1] = h2f((uint16_t)(b[w] >> 16));
     }
   }
+}
+
+// the value of another lane of the quad (kPerm: quad_perm selectors)
+template <int kPerm>
+__device__ __forceinline__ float quad_xor(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), kPerm, 0xF, 0xF, false));
 }
 
 // LDS needed by attend_range (floats)
@@ -88,15 +100,15 @@ __device__ __forceinline__ void attend_range(const uint16_t* __restrict__ q,
   }
   for (int t = kstart + w * 16 + quad; t < kend; t += 64) {
     float kx[16], vx[16];
-    load_row16(c.kc8, c.ksc, c.ktail, c.committed, t, kvh, d0, kx);
-    load_row16(c.vc8, c.vsc, c.vtail, c.committed, t, kvh, d0, vx);
+    load_row16(c.kc8, c.ksc, c.ktail, c.knew, c.fresh, c.committed, t, kvh, d0, kx);
+    load_row16(c.vc8, c.vsc, c.vtail, c.vnew, c.fresh, c.committed, t, kvh, d0, vx);
 #pragma unroll
     for (int j = 0; j < 4; j++) {
       float acc = 0.f;
 #pragma unroll
       for (int i = 0; i < 16; i++) acc = __builtin_fmaf(qr[j][i], kx[i], acc);
-      acc += __shfl_xor(acc, 1);
-      acc += __shfl_xor(acc, 2);
+      acc += quad_xor<0xB1>(acc);  // lane ^ 1
+      acc += quad_xor<0x4E>(acc);  // lane ^ 2
       const float s = acc * scale;
       const float mnew = __builtin_fmaxf(m[j], s);
       const float cc = fast_exp(m[j] - mnew), p = fast_exp(s - mnew);
@@ -112,29 +124,32 @@ __device__ __forceinline__ void attend_range(const uint16_t* __restrict__ q,
   float* sLw = sMw + 16;             // [4][4]
 #pragma unroll
   for (int j = 0; j < 4; j++) {
-    const float wm = wave_max(m[j]);
+    const float wm = wave_max_fast(m[j]);
     if (lane == 0) sMw[w * 4 + j] = wm;
   }
   __syncthreads();
+  // Sums over the wave's 16 quads without LDS permutes: four dims at once over
+  // the lanes {l, l ^ 16, l ^ 32, l ^ 48} (col4_sum4 leaves lane block b dim 4k
+  // + b), then rotations by 4 and 8 within the 16-lane rows.  (One permute
+  // step per dim and level, 256 a wave, was half of a short split's time.)
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     const float bm = __builtin_fmaxf(__builtin_fmaxf(sMw[j], sMw[4 + j]),
                                      __builtin_fmaxf(sMw[8 + j], sMw[12 + j]));
     const float alpha = fast_exp(m[j] - bm);
     float lj = l[j] * alpha;
-#pragma unroll
-    for (int off = 4; off <= 32; off <<= 1) lj += __shfl_xor(lj, off);
+    lj += row_ror<4>(lj);
+    lj += row_ror<8>(lj);
+    lj = col4_sum(lj);
     if (lane == 0) sLw[w * 4 + j] = lj;
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-      float v = o[j][i] * alpha;
-#pragma unroll
-      for (int off = 4; off <= 32; off <<= 1) v += __shfl_xor(v, off);
-      o[j][i] = v;
-    }
-    if (quad == 0) {
-#pragma unroll
-      for (int i = 0; i < 16; i++) sOw[(w * 4 + j) * D + d0 + i] = o[j][i];
+    for (int k = 0; k < 4; k++) {
+      float v = col4_sum4(o[j][4 * k] * alpha, o[j][4 * k + 1] * alpha, o[j][4 * k + 2] * alpha,
+                          o[j][4 * k + 3] * alpha);
+      v += row_ror<4>(v);
+      v += row_ror<8>(v);
+      // lanes 0..3 of each 16-lane row: part lane & 3, dim 4k + row
+      if ((lane & 12) == 0) sOw[(w * 4 + j) * D + d0 + 4 * k + (lane >> 4)] = v;
     }
     if (tid == 0) sM[j] = bm;
   }

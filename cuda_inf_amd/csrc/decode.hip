@@ -38,6 +38,14 @@ __global__ __launch_bounds__(256) void k_decode_split(const uint16_t* __restrict
     pm[pi] = sM[j];
     pl[pi] = sL[j];
   }
+  // the fresh token into its tail row (kv_write_tail, engine.cu:190-198), by
+  // the workgroup whose range holds it: no other one reads that row
+  if (c.fresh >= a && c.fresh < b && threadIdx.x < 16) {
+    const int x = threadIdx.x & 7;
+    const uint16_t* src = threadIdx.x < 8 ? c.knew : c.vnew;
+    uint16_t* dst = (uint16_t*)(threadIdx.x < 8 ? c.ktail : c.vtail);
+    *(u32x4*)(dst + ((size_t)(c.fresh - c.committed) * NKV + kvh) * D + 8 * x) = *(const u32x4*)(src + kvh * D + 8 * x);
+  }
 }
 
 // engine.cu:467-480 with runtime nsplit: the same merge (global max over the
@@ -191,7 +199,29 @@ static int decode_split(const uint16_t* q, const uint8_t* kc8, const uint8_t* vc
   if (nsplit <= kSplitMfmaMax && (qpos + nsplit) / nsplit >= kSplitMfmaMinKeys)
     return cia_split_mfma(q, kc8, vc8, ksc, vsc, ktail, vtail, committed, qpos, scale, pm, pl, po,
                           nsplit, ws, stream);
-  Group64Cache c{kc8, vc8, ksc, vsc, ktail, vtail, committed};
+  Group64Cache c{kc8, vc8, ksc, vsc, ktail, vtail, committed, nullptr, nullptr, -1};
+  hipLaunchKernelGGL(k_decode_split, dim3(NKV, nsplit), dim3(256), 0, (hipStream_t)stream, q, c,
+                     qpos, scale, pm, pl, po, nsplit);
+  return launch_status();
+}
+
+// A single-token step of a layer with nsplit > 0 whose splits take the fp32
+// kernel: the fresh token's tail write rides in the split launch.  Returns -1
+// where that kernel is not the one that runs or the arguments are not the
+// append's and the split's together (the caller then appends and splits, with
+// their own errors).  Internal entry of the layer driver; the step must not
+// fill the group.  (A step at 700 keys, 16 splits: 9.6 us with the append's own
+// launch, 7.9 so; 13.0 before attend_range's merge left the LDS permutes.)
+extern "C" __attribute__((visibility("hidden"))) int cia_decode_split_append(
+    const uint16_t* q, const uint8_t* kc8, const uint8_t* vc8, const uint16_t* ksc,
+    const uint16_t* vsc, uint16_t* ktail, uint16_t* vtail, const uint16_t* knew,
+    const uint16_t* vnew, int committed, int qpos, float scale, float* pm, float* pl, float* po,
+    int nsplit, void* stream) {
+  if (check_cache(q, kc8, vc8, ksc, vsc, ktail, vtail, committed) || !pm || !pl || !po ||
+      !aligned(knew, 16) || !aligned(vnew, 16) || nsplit < 1 || nsplit > CIA_NSPLIT_MAX ||
+      (nsplit <= kSplitMfmaMax && (qpos + nsplit) / nsplit >= kSplitMfmaMinKeys))
+    return -1;
+  Group64Cache c{kc8, vc8, ksc, vsc, ktail, vtail, committed, knew, vnew, qpos};
   hipLaunchKernelGGL(k_decode_split, dim3(NKV, nsplit), dim3(256), 0, (hipStream_t)stream, q, c,
                      qpos, scale, pm, pl, po, nsplit);
   return launch_status();

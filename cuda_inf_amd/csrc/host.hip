@@ -21,6 +21,12 @@ extern "C" __attribute__((visibility("hidden"))) int cia_decode_mfma(
     const uint16_t* vnew, int committed, int qpos, float scale, uint16_t* out, void* ws,
     int64_t ws_bytes, void* stream, void* mid_event, const void* prep);
 
+extern "C" __attribute__((visibility("hidden"))) int cia_decode_split_append(
+    const uint16_t* q, const uint8_t* kc8, const uint8_t* vc8, const uint16_t* ksc,
+    const uint16_t* vsc, uint16_t* ktail, uint16_t* vtail, const uint16_t* knew,
+    const uint16_t* vnew, int committed, int qpos, float scale, float* pm, float* pl, float* po,
+    int nsplit, void* stream);
+
 extern "C" __attribute__((visibility("hidden"))) int cia_h2o_decode_step(
     const uint16_t* q, const uint16_t* k, const uint16_t* v, uint8_t* kf, uint8_t* vf,
     uint16_t* ks, uint16_t* vs, float* attn_sum, int32_t* slot_pos, int32_t* dst_slots,
@@ -293,6 +299,31 @@ int decode_fused_append(cia_layer* L, const uint16_t* q, const uint16_t* k, cons
   return st;
 }
 
+// One token of a layer with nsplit > 0 (q, k prepared): append and attend.  A
+// token that lands in the tail without filling it is written by the split
+// launch itself where the fp32 split kernel runs (one launch of three saved).
+// ev: recorded before the attention launches and after the first of them
+int split_step(cia_layer* L, const uint16_t* q, const uint16_t* k, const uint16_t* v,
+               uint16_t* out, int past, float scale, void* stream, void* ev0 = nullptr,
+               void* mid = nullptr) {
+  hipStream_t s = (hipStream_t)stream;
+  const int slot = past - L->committed;
+  int st;
+  if (L->nsplit > 0 && slot >= 0 && slot < CIA_KVGROUP - 1 && past < L->maxT && out) {
+    if (ev0 && (st = hip_check(hipEventRecord((hipEvent_t)ev0, s)))) return st;
+    st = cia_decode_split_append(q, L->kc8, L->vc8, L->ksc, L->vsc, L->ktail, L->vtail, k, v,
+                                 L->committed, past, scale, L->pm, L->pl, L->po, L->nsplit, stream);
+    if (st > 0) return st;
+    if (st == 0) {
+      if (mid && (st = hip_check(hipEventRecord((hipEvent_t)mid, s)))) return st;
+      return cia_attn_decode_combine(L->pm, L->pl, L->po, out, L->nsplit, stream);
+    }
+  }
+  if ((st = group64_append(L, k, v, 1, past, stream))) return st;
+  if (ev0 && (st = hip_check(hipEventRecord((hipEvent_t)ev0, s)))) return st;
+  return group64_attend(L, q, out, 1, past, scale, stream, mid);
+}
+
 }  // namespace
 
 extern "C" int cia_layer_forward(cia_layer* L, const uint16_t* q, const uint16_t* k,
@@ -307,6 +338,7 @@ extern "C" int cia_layer_forward(cia_layer* L, const uint16_t* q, const uint16_t
   if (S == 1 && fused_append_ok(L, past))
     return decode_fused_append(L, q, k, v, out, past, scale, stream);
   if ((st = prep_qk(L, q, k, S, past, stream))) return st;
+  if (S == 1) return split_step(L, q, k, v, out, past, scale, stream);
   st = group64_append(L, k, v, S, past, stream);
   if (st) return st;
   return group64_attend(L, q, out, S, past, scale, stream);
@@ -410,16 +442,15 @@ extern "C" int cia_decode_loop_runs(cia_layer* layers, int n_layers, const uint1
       const bool fused = fused_append_ok(L, pos);
       const uint16_t* qi = q + r * qrow;
       const uint16_t* ki = k + r * krow;
-      if (!fused) {
-        if ((st = prep_qk(L, qi, ki, 1, pos, stream))) return st;
-        st = group64_append(L, ki, v + r * krow, 1, pos, stream);
-        if (st) return st;
-      }
       void* mid = events ? events[3 * r + 1] : nullptr;
-      if (events && (st = hip_check(hipEventRecord((hipEvent_t)events[3 * r], s)))) return st;
-      st = fused ? decode_fused_append(L, qi, ki, v + r * krow, out + r * qrow, pos, scale,
-                                       stream, mid)
-                 : group64_attend(L, qi, out + r * qrow, 1, pos, scale, stream, mid);
+      if (fused) {
+        if (events && (st = hip_check(hipEventRecord((hipEvent_t)events[3 * r], s)))) return st;
+        st = decode_fused_append(L, qi, ki, v + r * krow, out + r * qrow, pos, scale, stream, mid);
+      } else {
+        if ((st = prep_qk(L, qi, ki, 1, pos, stream))) return st;
+        st = split_step(L, qi, ki, v + r * krow, out + r * qrow, pos, scale, stream,
+                        events ? events[3 * r] : nullptr, mid);
+      }
       if (st) return st;
       if (events && (st = hip_check(hipEventRecord((hipEvent_t)events[3 * r + 2], s)))) return st;
       l++;

@@ -208,6 +208,35 @@ def test_prefill_shapes(orc, cia, dev, S, past):
         assert_close_f16(_u16(out), r32)
 
 
+@pytest.mark.parametrize("nsplit,n0", [(16, 0), (16, 700), (64, 100), (600, 1980)])
+def test_split_steps_append_in_launch(orc, cia, dev, nsplit, n0):
+    """Single-token steps of a layer with nsplit > 0 on the fp32 split kernel,
+    which writes the fresh token's tail row itself: from an empty cache, with
+    more splits than keys, and across a group fill (that step appends in a
+    launch of its own).  Tail rows and committed bytes are those of the
+    append, and the rows past the last token stay as they were."""
+    from cuda_inf_amd.layer import AttnLayer
+    from cuda_inf_amd.workload import qkv
+    L = AttnLayer(n0 + 200, nsplit=nsplit, device=dev)
+    ref = orc.Group64Cache(n0 + 200)
+    if n0:
+        q0, k0, v0 = qkv(n0, seed=31, device="cpu", outliers=True)
+        L.forward(q0.to(dev), k0.to(dev), v0.to(dev), 0)
+        ref.append(_u16(k0), _u16(v0), 0)
+    for j in range(70):
+        q, k, v = qkv(1, seed=500 + j, device="cpu", past=n0 + j, outliers=True)
+        out, _ = L.forward(q.to(dev), k.to(dev), v.to(dev), n0 + j)
+        ref.append(_u16(k), _u16(v), n0 + j)
+        torch.cuda.synchronize()
+        assert L.committed == ref.committed
+        n = n0 + j + 1 - ref.committed
+        assert np.array_equal(_u16(L.ktail)[:n], ref.ktail[:n]), f"K tail at step {j}"
+        assert np.array_equal(_u16(L.vtail)[:n], ref.vtail[:n]), f"V tail at step {j}"
+        assert np.array_equal(L.kc8.cpu().numpy(), ref.kc8), f"K bytes at step {j}"
+        _, r32, _ = orc.attn_decode(_u16(q), ref, n0 + j, nsplit=nsplit)
+        assert_close_f16(_u16(out)[0], r32, what=f"step {j}")
+
+
 def test_decode_steps_through_commit(orc, cia, dev):
     """Decode steps that cross a group boundary (tail fills, commit, new tail)."""
     from cuda_inf_amd.layer import AttnLayer
