@@ -450,6 +450,172 @@ __global__ __launch_bounds__(64 * kGemmWaves) void k_gemm_int4(GemvArgs a) {
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
 }
 
+// ---------------------------------------------------------------- large tiles
+// The tile kernel's group step is bound by vector work and LDS reads as much as
+// by its products: a wave dequantises 32 columns for 64 rows.  Here a wave has
+// 128 rows x (16 kNT) columns of a 256 x (64 kNT) workgroup tile, so a
+// dequantised operand serves twice the rows, and the columns' scales come from
+// an LDS table filled once (fetched per group, 8 waves x 64 two-byte loads in
+// different rows cost the step 500 cycles of address work).  Two slots: the
+// next group's DMA goes out after the barrier that ends the last group and has
+// the whole step to land.  Layouts, the order of k and the sums are the tile
+// kernel's: the same bits.  K up to 2048 (the LDS).
+// (q/k/v of 4096 rows, kNT = 3, one round of 256 workgroups: 77 -> 58 us, 885
+// TFLOP/s; out_proj, kNT = 2: 66 -> 51.)
+constexpr int kBigRows = 256;
+constexpr int kBigMaxK = 2048;
+
+// grid = the tiles, ceil(rows / (64 kNT)) * ceil(M / 256), up to a multiple of 8;
+// block = 512
+template <int kOut, int kNT>
+__global__ __launch_bounds__(64 * kGemmWaves) void k_gemm_int4_big(GemvArgs a) {
+  constexpr int kCols = 64 * kNT, kXB = kBigRows * 256, kWB = kCols * 64, kSlotB = kXB + kWB;
+  __shared__ __attribute__((aligned(16))) uint8_t lds[2 * kSlotB + (kBigMaxK / 128) * kCols * 2];
+  const int tid = threadIdx.x, l = tid & 63, n16 = l & 15, q = l >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), wm = w >> 2, wn = w & 3;
+  // Workgroups go to the 8 XCDs in turn: XCD x takes the tiles x gridDim.x / 8
+  // on, row tiles slowest, so that its L2 sees a few row blocks of x and not
+  // all of it.
+  const int nct = (a.rows + kCols - 1) / kCols;
+  const int tile = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const int m0 = tile / nct * kBigRows, r0 = tile % nct * kCols;
+  if (m0 >= a.M) return;
+  const int K = a.K, ng = K >> 7;
+  uint16_t* ssc = (uint16_t*)(lds + 2 * kSlotB);  // [group][column]
+  // DMA sources: X instruction t of wave w fills rows 4 (8w + t) .. + 3, as the
+  // tile kernel's; W instruction u columns 16 u .. + 15, u = w and w + 8
+  const uint8_t* xsrc[8];
+#pragma unroll
+  for (int t = 0; t < 8; t++) {
+    const int r = 4 * (8 * w + t) + (l >> 4), m = m0 + r;
+    xsrc[t] = (const uint8_t*)(a.x + (size_t)(m < a.M ? m : a.M - 1) * K) + 16 * ((l & 15) ^ xsw(r));
+  }
+  const uint8_t* wsrc[2];
+#pragma unroll
+  for (int t = 0; t < 2; t++) {
+    const int c = 16 * (w + 8 * t) + (l >> 2);
+    wsrc[t] = col_packed(a, col_ref(a, r0 + (c < kCols ? c : 0)), K) + 16 * ((l & 3) ^ ((c >> 2) & 3));
+  }
+  auto issue = [&](int g) __attribute__((always_inline)) {
+    uint8_t* slot = lds + (g & 1) * kSlotB;
+#pragma unroll
+    for (int t = 0; t < 8; t++)
+      __builtin_amdgcn_global_load_lds((gbl_void_t*)(xsrc[t] + 256 * g),
+                                       (lds_void_t*)(slot + (8 * w + t) * 1024), 16, 0, 0);
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+      if (w + 8 * t < 4 * kNT)
+        __builtin_amdgcn_global_load_lds((gbl_void_t*)(wsrc[t] + 64 * g),
+                                         (lds_void_t*)(slot + kXB + (w + 8 * t) * 1024), 16, 0, 0);
+  };
+  issue(0);
+  // 16 neighbouring threads read a column's scales
+#pragma unroll
+  for (int e0 = 0; e0 < 16 * kCols; e0 += 64 * kGemmWaves) {
+    const int c = (e0 + tid) >> 4, g = tid & 15;
+    if (g < ng) ssc[g * kCols + c] = col_scales(a, col_ref(a, r0 + c), K)[g];
+  }
+  f32x4 C[8][kNT];
+#pragma unroll
+  for (int i = 0; i < 8; i++)
+#pragma unroll
+    for (int j = 0; j < kNT; j++) C[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int g = 0; g < ng; g++) {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0): this wave's DMA (and scales) landed
+    __builtin_amdgcn_s_barrier();        // every wave's did; the other slot is read
+    asm volatile("" ::: "memory");
+    if (g + 1 < ng) issue(g + 1);
+    const uint8_t* slot = lds + (g & 1) * kSlotB;
+    const uint16_t* xs = (const uint16_t*)slot + (128 * wm + n16) * 128;
+    // Units of two row tiles x two k steps, in order: a unit's x operands are
+    // requested before the products of the unit before it, and the columns of
+    // its k steps are dequantised where the row tiles first need them.
+    f16x8 A[2][4];
+    auto load_a = [&](int u, f16x8 (&o)[4]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+          o[2 * i + s] = *(const f16x8*)(xs + 16 * (2 * (u >> 1) + i) * 128 +
+                                         8 * ((4 * q + 2 * (u & 1) + s) ^ xsw(n16)));
+    };
+    u32x4 wq[kNT];
+    float scl[kNT];
+#pragma unroll
+    for (int j = 0; j < kNT; j++) {
+      const int c = 16 * (kNT * wn + j) + n16;
+      wq[j] = *(const u32x4*)(slot + kXB + c * 64 + 16 * (q ^ ((c >> 2) & 3)));
+      scl[j] = h2f(ssc[g * kCols + c]);
+    }
+    load_a(0, A[0]);
+    f16x8 B[kNT][4];
+    f32x4 P[2][2][kNT];  // of a pair of row tiles, and of the pair before
+    auto scale_add = [&](int pr) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < kNT; j++)
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+            C[2 * pr + i][j][e] = __builtin_fmaf(P[pr & 1][i][j][e], scl[j], C[2 * pr + i][j][e]);
+    };
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      if (u + 1 < 8) load_a(u + 1, A[(u + 1) & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+      const int s0 = 2 * (u & 1), pr = u >> 1;
+      if (u < 2)
+#pragma unroll
+        for (int j = 0; j < kNT; j++) {
+          B[j][s0] = nib8(wq[j][s0]);
+          B[j][s0 + 1] = nib8(wq[j][s0 + 1]);
+        }
+#pragma unroll
+      for (int s = 0; s < 2; s++)
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+          for (int j = 0; j < kNT; j++)
+            P[pr & 1][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                A[u & 1][2 * i + s], B[j][s0 + s], s0 + s == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : P[pr & 1][i][j], 0, 0, 0);
+      // the pair before is scaled between this pair's first products
+      if (pr > 0 && (u & 1) == 0) {
+        scale_add(pr - 1);
+#pragma unroll
+        for (int k = 0; k < 4 * kNT; k++) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
+          __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // two vector instructions
+        }
+      }
+    }
+    scale_add(3);
+  }
+  // outputs, as the tile kernel's, a column's 32 rows at a time
+#pragma unroll
+  for (int j = 0; j < kNT; j++) {
+    const int col = r0 + 16 * (kNT * wn + j) + n16;
+    const OutCol<kOut> o(a, col);
+    float yo[8][4];
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int m = m0 + 128 * wm + 16 * i + 4 * q + e;
+        yo[i][e] = o.old(m < a.M ? m : a.M - 1);
+      }
+    if (col < a.rows) {
+#pragma unroll
+      for (int i = 0; i < 8; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int m = m0 + 128 * wm + 16 * i + 4 * q + e;
+          if (m < a.M) o.put(m, C[i][j][e], yo[i][e]);
+        }
+    }
+  }
+}
+
 // ---------------------------------------------------------------- K-split GEMM
 // A few to about a thousand rows of x (short prompts, chat turns): too few
 // 128 x 128 tiles to fill the chip, and each tile's 16 scale groups a serial
@@ -646,6 +812,19 @@ static float ks_time(const KsShape& k, int M, int rows) {
 }
 
 // the matrix-core kernels, by the launch's output form
+// Time of a tiling of many rows: rounds of 256 workgroups (one a compute unit)
+// times a tile's own time, 128 x 128 = 100.  (One round / two, K = 2048: 128 x
+// 128 29 / 51 us, 256 x 128 35 / 72, 256 x 192 46 to 58.  q/k/v of 1024 rows:
+// 128 x 128 29 us, the others 35 and 46; 2048 rows: 51, 39 and 51; 3000: 74,
+// 71 and 52.  out_proj of 2048 rows: 36, 46 and 61; 3000: 59, 48 and 62.)  The
+// sums are the same in each, so the choice may depend on the rows of W.
+static long tile_count(const GemvArgs& a, int cols, int xrows) {
+  return (a.rows + (long)cols - 1) / cols * ((a.M + (long)xrows - 1) / xrows);
+}
+static long big_time(const GemvArgs& a, int cols, int xrows, int cost) {
+  return (tile_count(a, cols, xrows) + 255) / 256 * cost;
+}
+
 template <int kOut>
 static void gemm_launch(const GemvArgs& a, hipStream_t s) {
   if (a.M < kTileMinM && a.K <= kKsMaxK) {
@@ -662,8 +841,23 @@ static void gemm_launch(const GemvArgs& a, hipStream_t s) {
       case 44: return ks_launch<kOut, 4, 4>(a, s);
     }
   }
+  const dim3 block(64 * kGemmWaves);
+  if (a.K <= kBigMaxK) {
+    const long t = big_time(a, kTile, kTile, 100), t2 = big_time(a, 128, kBigRows, 145),
+               t3 = big_time(a, 192, kBigRows, 200);
+    const int n2 = (int)(tile_count(a, 128, kBigRows) + 7) / 8 * 8,
+              n3 = (int)(tile_count(a, 192, kBigRows) + 7) / 8 * 8;
+    if (t2 < t && t2 <= t3) {
+      hipLaunchKernelGGL((k_gemm_int4_big<kOut, 2>), dim3(n2), block, 0, s, a);
+      return;
+    }
+    if (t3 < t) {
+      hipLaunchKernelGGL((k_gemm_int4_big<kOut, 3>), dim3(n3), block, 0, s, a);
+      return;
+    }
+  }
   hipLaunchKernelGGL(k_gemm_int4<kOut>, dim3((unsigned)((a.rows + kTile - 1) / kTile),
-                     (unsigned)((a.M + kTile - 1) / kTile)), dim3(64 * kGemmWaves), 0, s, a);
+                     (unsigned)((a.M + kTile - 1) / kTile)), block, 0, s, a);
 }
 
 template <int kM>

@@ -127,8 +127,21 @@ def test_gemm_ksplit(orc, cia, dev, N, K, M, seed):
     test_gemv_int4(orc, cia, dev, N, K, M, "normal", seed)
 
 
-@pytest.mark.parametrize("M,seed", [(2, 31), (16, 32), (40, 33), (300, 34)])
-def test_qkv_ksplit_bits(orc, cia, dev, M, seed):
+# The 256-row tiles (more than 768 rows of x, K up to 2048, where they need
+# fewer rounds of 256 workgroups): 128 and 192 columns a tile, each with ragged
+# last rows and columns and tiles past the end of the grid; one, three and
+# sixteen groups; the first K past the limit, and the last rows of 128 x 128.
+BIG_TILES = [(2080, 128, 2060, 40), (2080, 384, 2060, 41), (4100, 256, 2561, 42),
+             (1100, 2048, 4000, 43), (2080, 2176, 2060, 44), (2048, 128, 2048, 45)]
+
+
+@pytest.mark.parametrize("N,K,M,seed", BIG_TILES)
+def test_gemm_big_tiles(orc, cia, dev, N, K, M, seed):
+    test_gemv_int4(orc, cia, dev, N, K, M, "normal", seed)
+
+
+@pytest.mark.parametrize("M,seed", [(2, 31), (16, 32), (40, 33), (300, 34), (1600, 35), (2600, 36)])
+def test_qkv_shapes_bits(orc, cia, dev, M, seed):
     """q/k/v in one launch have the bits of the three matrices alone,
     whatever tile shapes the launches take."""
     test_qkv_proj_int4(orc, cia, dev, M, seed)
