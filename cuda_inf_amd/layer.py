@@ -15,7 +15,7 @@ import torch
 from . import _lib
 from ._lib import (D, KVGROUP, NH, NKV, NSPLIT_DEFAULT, call, cia_append_op, cia_attn_proj,
                    cia_layer)
-from .kernels import decode_workspace_bytes, h2o_workspace_bytes
+from .kernels import decode_workspace_bytes, h2o_workspace_bytes, stream_handle
 
 HIDDEN = _lib.HIDDEN
 
@@ -151,7 +151,7 @@ class AttnLayer:
         ev = ctypes.c_int(-1)
         call("cia_layer_forward", ctypes.byref(self._s), q.data_ptr(), k.data_ptr(), v.data_ptr(),
              out.data_ptr(), S, past, float(scale), ctypes.byref(ev) if evicted else None,
-             torch.cuda.current_stream().cuda_stream)
+             stream_handle())
         return out, (ev.value if evicted else None)
 
     # -------------------------------------------------------- projections
@@ -191,7 +191,7 @@ class AttnLayer:
         ev = ctypes.c_int(-1)
         call("cia_attn_block_forward", ctypes.byref(self._s), ctypes.byref(self._p), x.data_ptr(),
              h.data_ptr(), S, past, float(scale), ctypes.byref(ev) if evicted else None,
-             torch.cuda.current_stream().cuda_stream)
+             stream_handle())
         return ev.value if evicted else None
 
 
@@ -209,7 +209,7 @@ def attn_block_loop(layers, x, h, past: int, steps: int, scale: float = 0.125, e
         ev = (ctypes.c_void_p * len(events))(*[e.cuda_event for e in events])
     try:
         call("cia_attn_block_loop", arr, parr, n, x.data_ptr(), h.data_ptr(), past, steps,
-             float(scale), ev, torch.cuda.current_stream().cuda_stream)
+             float(scale), ev, stream_handle())
     finally:
         for L, s in zip(layers, arr):  # host counters advance in the copies
             L._s.committed, L._s.n_live = s.committed, s.n_live

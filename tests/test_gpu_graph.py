@@ -135,3 +135,44 @@ def test_decode_loop_replay_bit_identical(orc, cia, dev):
             assert la.committed == lb.committed
             for n in names:
                 assert torch.equal(getattr(la, n), getattr(lb, n)), (r, n)
+
+
+@pytest.mark.parametrize("kind", ["default", "side", "external", "thread", "capture"])
+def test_stream_handle_is_the_current_stream(dev, kind):
+    """The handle the Python calls pass on is torch's current stream: the
+    default one, a side stream, an external one, another thread's own, and the
+    capturing one."""
+    import threading
+    from cuda_inf_amd.kernels import stream_handle
+
+    def same():
+        return stream_handle() == torch.cuda.current_stream().cuda_stream
+
+    side = torch.cuda.Stream()
+    if kind == "default":
+        assert same()
+    elif kind == "capture":
+        g, x = torch.cuda.CUDAGraph(), torch.zeros(8, device=dev)
+        with torch.cuda.graph(g, stream=side):
+            ok, h = same(), stream_handle()
+            x.add_(1)
+        assert ok and h == side.cuda_stream
+    elif kind == "thread":
+        got = []
+
+        def work():
+            got.append((same(), stream_handle()))
+            with torch.cuda.stream(side):
+                got.append((same(), stream_handle()))
+
+        with torch.cuda.stream(torch.cuda.Stream()):
+            t = threading.Thread(target=work)
+            t.start()
+            t.join()
+            assert same()
+        assert all(ok for ok, _ in got) and got[1][1] == side.cuda_stream
+    else:
+        s = side if kind == "side" else torch.cuda.ExternalStream(side.cuda_stream)
+        with torch.cuda.stream(s):
+            assert same() and stream_handle() == side.cuda_stream
+        assert same()
