@@ -129,19 +129,59 @@ def test_gemm_ksplit(orc, cia, dev, N, K, M, seed):
 
 # The 256-row tiles (more than 768 rows of x, K up to 2048, where they need
 # fewer rounds of 256 workgroups): 128 and 192 columns a tile, each with ragged
-# last rows and columns and tiles past the end of the grid; one, three and
-# sixteen groups; the first K past the limit, and the last rows of 128 x 128.
-BIG_TILES = [(2080, 128, 2060, 40), (2080, 384, 2060, 41), (4100, 256, 2561, 42),
-             (1100, 2048, 4000, 43), (2080, 2176, 2060, 44), (2048, 128, 2048, 45)]
+# last rows and columns and tiles past the end of the grid; one, two, three and
+# sixteen groups.  Their sums are in the 128 x 128 tiles' order, so the rows
+# have the bits of launches over slices of them that take those; the first and
+# last rows are checked against the oracle.
+BIG_TILES = [(2080, 128, 2060, 2, 40), (2080, 384, 2060, 2, 41), (4100, 256, 2561, 3, 42),
+             (1100, 2048, 4000, 4, 43), (3072, 2048, 2700, 3, 44)]
 
 
-@pytest.mark.parametrize("N,K,M,seed", BIG_TILES)
-def test_gemm_big_tiles(orc, cia, dev, N, K, M, seed):
-    test_gemv_int4(orc, cia, dev, N, K, M, "normal", seed)
+@pytest.mark.parametrize("N,K,M,parts,seed", BIG_TILES)
+def test_gemm_big_tiles(orc, cia, dev, N, K, M, parts, seed):
+    from cuda_inf_amd import kernels as KK
+    rng = np.random.default_rng(seed)
+    packed, scales = _weights(rng, N, K, orc, "normal")
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    xd, pd, sd = _t(x, dev), _t(packed, dev), _t(scales, dev)
+    print(f"big tiles N={N} K={K} M={M}", flush=True)
+    for add in (False, True):
+        y0 = torch.full((M, N), 0.5 if add else float("nan"), dtype=torch.float32, device=dev)
+        y, z = y0.clone(), y0.clone()
+        KK.gemv_int4(xd, pd, sd, y, N, K, M, add=add)
+        for r in torch.arange(M).tensor_split(parts):
+            r0, n = int(r[0]), len(r)
+            assert n > 768
+            KK.gemv_int4(xd[r0:r0 + n], pd, sd, z[r0:r0 + n], N, K, n, add=add)
+        torch.cuda.synchronize()
+        assert torch.equal(y, z)
+        if not add:
+            ends = np.r_[0:3, M - 3:M]
+            ref, ab = orc.gemv_int4(x[ends], packed, scales, want_absum=True)
+            _check(y.cpu().numpy()[ends], ref, ab, "y")
 
 
-@pytest.mark.parametrize("M,seed", [(2, 31), (16, 32), (40, 33), (300, 34), (1600, 35), (2600, 36)])
+@pytest.mark.parametrize("M,seed", [(2, 31), (16, 32), (40, 33), (300, 34)])
 def test_qkv_shapes_bits(orc, cia, dev, M, seed):
     """q/k/v in one launch have the bits of the three matrices alone,
     whatever tile shapes the launches take."""
     test_qkv_proj_int4(orc, cia, dev, M, seed)
+
+
+@pytest.mark.parametrize("M,seed", [(1600, 35), (2700, 36)])
+def test_qkv_big_tiles_bits(orc, cia, dev, M, seed):
+    """The same for the 256-row tiles of 128 and 192 columns: the fp16
+    rounding of each matrix's own fp32 sums, bit for bit."""
+    from cuda_inf_amd import kernels as KK
+    rng = np.random.default_rng(seed)
+    K, rows = 2048, {"q": 2048, "k": 512, "v": 512}
+    W = {n: tuple(_t(a, dev) for a in _weights(rng, N, K, orc)) for n, N in rows.items()}
+    x = _t((rng.standard_normal((M, K)) * 0.5).astype(np.float16), dev)
+    out = {n: torch.zeros((M, N), dtype=torch.float16, device=dev) for n, N in rows.items()}
+    print(f"qkv big tiles M={M}", flush=True)
+    KK.qkv_proj_int4(x, W["q"], W["k"], W["v"], out["q"], out["k"], out["v"], M, K)
+    for n, N in rows.items():
+        y = torch.zeros((M, N), dtype=torch.float32, device=dev)
+        KK.gemv_int4(x, *W[n], y, N, K, M)
+        torch.cuda.synchronize()
+        assert torch.equal(out[n].view(torch.int16), y.half().view(torch.int16)), n
