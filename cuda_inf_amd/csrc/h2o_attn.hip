@@ -581,8 +581,8 @@ __global__ __launch_bounds__(1024) void k_h2o_mass(H2oArgs a, int nsw) {
 // Queries that see no slot of a block or workgroup are passed over; a product
 // of a slot that its query does not see is -0, which leaves any sum as it is.
 // (S = 1024 into an empty 2048-slot buffer: per 16 queries a scores and a mass
-// launch, its chain on one workgroup per 256 slots, 2500 us in all; as here 300:
-// stats 81, weights 7, chain 179, outputs 28.)
+// launch, its chain on one workgroup per 256 slots, 2500 us in all; as here 277.  By
+// the launch: stats 76, weights 7, chain 178, outputs 28.)
 struct MassArgs {
   const uint16_t* q;  // first query row of the chunk
   const uint8_t* kf;
@@ -600,6 +600,10 @@ struct MassArgs {
 // 64 136 / 37.)
 constexpr int kManyMin = 16;
 constexpr int kStQ = 4;  // queries of a stats group
+
+// half a q row in the constant address space
+typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
+typedef __attribute__((address_space(4))) u32x16 __attribute__((aligned(16))) q16_t;
 
 // 16-byte piece swizzle of K row r in a wave's LDS: each lane then reads one
 // whole row, and lanes r, r + 4, .. of a bank window take distinct pieces
@@ -622,34 +626,26 @@ __device__ __forceinline__ void key_row(const u32x4 (&w)[4], float ksc, float (&
 // grid = (2 nblk, ceil(nq / (kStQ ngrp))), block = 256: wave w, kv head 4
 // (blockIdx.x & 1) + w, ngrp groups of kStQ queries
 __global__ __launch_bounds__(256) void k_h2o_stats(MassArgs a, int ngrp) {
-  __shared__ __attribute__((aligned(16))) uint8_t lds[4][64 * D + kStQ * GQA * D * 2];
+  __shared__ __attribute__((aligned(16))) uint8_t lds[4][64 * D];
   const int wv = wave_id(), lane = threadIdx.x & 63;
   // (the block rotates with the query group: workgroups go to the XCDs by their
   // number, and in a prompt the first blocks are seen by the most queries)
   const int blk = ((blockIdx.x >> 1) + blockIdx.y) % a.nblk, g = 4 * (blockIdx.x & 1) + wv;
   const int ib = blockIdx.y * kStQ * ngrp, ie = min(ib + kStQ * ngrp, a.nq);
   uint8_t* kl = lds[wv];
-  uint16_t* ql = (uint16_t*)(kl + 64 * D);
   const int t0 = blk * 64, t = t0 + lane;
   const bool live = t < a.n_live;
   const int tc = live ? t : a.n_live - 1;
   const int sp = live ? a.slot_pos[tc] : 0x7FFFFFFF;
   const uint16_t ks16 = a.ks[(size_t)tc * NKV + g];
   // the block's K rows, 4 neighbouring lanes to a row (rows past the last
-  // slot read it again), through LDS to one row a lane; q beside them (32
-  // lanes to a query's 4 heads), a group ahead
-  u32x4 kr[4], qr[kStQ / 2];
+  // slot read it again), through LDS to one row a lane
+  u32x4 kr[4];
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     const int r = min(t0 + 16 * j + (lane >> 2), a.n_live - 1);
     kr[j] = *(const u32x4*)(a.kf + ((size_t)r * NKV + g) * D + 16 * (lane & 3));
   }
-  auto load_q = [&](int i0) __attribute__((always_inline)) {
-#pragma unroll
-    for (int j = 0; j < kStQ / 2; j++)
-      qr[j] = *(const u32x4*)(a.q + ((size_t)min(i0 + 2 * j + (lane >> 5), a.nq - 1) * NH + g * GQA) * D + 8 * (lane & 31));
-  };
-  load_q(ib);
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     const int r = 16 * j + (lane >> 2);
@@ -660,45 +656,43 @@ __global__ __launch_bounds__(256) void k_h2o_stats(MassArgs a, int ngrp) {
   for (int p = 0; p < 4; p++) w[p] = *(const u32x4*)(kl + lane * 64 + 16 * (p ^ ksw(lane)));
   float k[D];
   key_row(w, h2f(ks16), k);
+  int i = ib;
+  for (; i < ie && !__any(sp <= a.qpos0 + i); i++)  // (positions rise with i)
+    if (lane < GQA) a.ml[(size_t)blk * (a.nq * NH) + i * NH + g * GQA + lane] = f32x2{kNegInf, 0.0f};
+  // A q row is the same for every lane: it comes through the scalar cache into
+  // 32 scalar registers, the next head's while this one's products are taken.
+  // (Read back from LDS by every lane, a row's 8 reads of 1 KB were as much LDS
+  // time as the products' issue: 81 us in the prompt above, 76 so.)
+  u32x16 qs[2][2];
+  auto load_q = [&](int n, u32x16 (&o)[2]) __attribute__((always_inline)) {  // head n of query i on
+    const int in = min(i + (n >> 2), ie - 1);
+    const auto* p = (const q16_t*)(uintptr_t)(a.q + ((size_t)in * NH + g * GQA + (n & 3)) * D);
+    o[0] = p[0];
+    o[1] = p[1];
+  };
+  if (i < ie) load_q(0, qs[0]);
 #pragma unroll 1
-  for (int i = ib; i < ie; i++) {
-    const int r = (i - ib) % kStQ;
-    if (r == 0) {
-#pragma unroll
-      for (int j = 0; j < kStQ / 2; j++) *(u32x4*)(ql + 512 * j + 8 * lane) = qr[j];
-      if (i + kStQ < ie) load_q(i + kStQ);
-    }
+  for (; i < ie; i++) {
     f32x2* ml = a.ml + (size_t)blk * (a.nq * NH) + i * NH + g * GQA;
     const bool ok = sp <= a.qpos0 + i;
-    if (!__any(ok)) {
-      if (lane < GQA) ml[lane] = f32x2{kNegInf, 0.0f};
-      continue;
-    }
-    // (two heads at a time: their q rows are what the registers hold beside k)
-#pragma unroll 1
-    for (int h0 = 0; h0 < GQA; h0 += 2) {
-      const uint16_t* q = ql + (r * GQA + h0) * D;
-      float s[2] = {0.0f, 0.0f};
+    f32x2 o = f32x2{0.0f, 0.0f};
 #pragma unroll
-      for (int d = 0; d < D; d += 8)
+    for (int h = 0; h < GQA; h++) {
+      u32x16(&qc)[2] = qs[h & 1];
+      asm volatile("" : "+s"(qc[0]), "+s"(qc[1]));  // (arrived: scalar loads have no order to wait by)
+      load_q(h + 1, qs[(h + 1) & 1]);
+      float s = 0.0f;
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-          const u32x4 qq = *(const u32x4*)(q + h * D + d);
-#pragma unroll
-          for (int x = 0; x < 4; x++) {
-            s[h] = __builtin_fmaf(h2f((uint16_t)qq[x]), k[d + 2 * x], s[h]);
-            s[h] = __builtin_fmaf(h2f((uint16_t)(qq[x] >> 16)), k[d + 2 * x + 1], s[h]);
-          }
-        }
-      f32x2 o[2];
-#pragma unroll
-      for (int h = 0; h < 2; h++) {
-        s[h] = ok ? s[h] * a.scale : kNegInf;
-        const float mb = wave_max_fast(s[h]);
-        o[h] = f32x2{mb, wave_tree_sum(ok ? exp_det(s[h] - mb) : 0.0f)};
+      for (int d = 0; d < D; d += 2) {
+        const uint32_t x = qc[d >> 5][(d & 31) >> 1];
+        s = __builtin_fmaf(h2f((uint16_t)x), k[d], s);
+        s = __builtin_fmaf(h2f((uint16_t)(x >> 16)), k[d + 1], s);
       }
-      if (lane < 2) ml[h0 + lane] = lane == 0 ? o[0] : o[1];
+      s = ok ? s * a.scale : kNegInf;
+      const float mb = wave_max_fast(s), l = wave_tree_sum(ok ? exp_det(s - mb) : 0.0f);
+      if (lane == h) o = f32x2{mb, l};
     }
+    if (lane < GQA) ml[lane] = o;
   }
 }
 
