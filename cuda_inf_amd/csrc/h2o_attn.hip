@@ -569,8 +569,8 @@ __global__ __launch_bounds__(1024) void k_h2o_mass(H2oArgs a, int nsw) {
 // for any number of queries (the outputs come from the matrix cores, in a
 // launch of their own, prefill_split.hip):
 //   k_h2o_stats    m_b and l_b: a wave holds a block's 64 keys of one kv head
-//                  in registers, lane = slot, for kStQ queries; q comes from
-//                  LDS by broadcast and enters the fma as fp16.
+//                  in registers, lane = slot, for kStQ queries; q, the same
+//                  for every lane, in scalar registers, fp16 into the fma.
 //   k_h2o_weights  w_b in place of l_b, lane = (query, head) row.
 //   k_h2o_chain    a workgroup per kSl slots: eight waves, one per kv head,
 //                  take s again and the products p = exp_det(s - m_b) w_b, lane

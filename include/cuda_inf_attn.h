@@ -264,7 +264,8 @@ int cia_h2o_place(const uint16_t* k, const uint16_t* v, uint8_t* kf,
  *   l = sum of l_b * c_b in ascending b; p = e * (c_b * (1/l));
  *   attn_sum[t] += p in (query, head) order.
  * ws: device scratch of ws_bytes >= cia_h2o_workspace_bytes(S, n_live)
- * bytes (16-byte aligned); queries are processed 16 at a time through it. */
+ * bytes (16-byte aligned); queries go through it in runs of as many as it
+ * holds, at least 16. */
 int cia_attention_h2o(const uint16_t* q, const uint8_t* kf, const uint8_t* vf,
                       const uint16_t* ks, const uint16_t* vs,
                       const int32_t* slot_pos, int n_live, uint16_t* out,
