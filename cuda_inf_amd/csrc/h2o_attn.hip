@@ -43,6 +43,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "h2o_chain.h"
 #include "h2o_place.h"
 
 namespace cia {
@@ -799,21 +800,22 @@ __global__ __launch_bounds__(64 * (NKV + 1)) void k_h2o_chain(MassArgs a) {
   // (query, head)'s piece p lies at p ^ (row & 7)) and (m_b, w_b), one step ahead
   constexpr int kPc = kQB / 16;  // pieces: 32 a query
   constexpr int kLd = (kPc + 63) / 64;
-  // (buffer loads: one lane offset for every step, rows past the chunk read 0)
+  // (buffer loads: rows past the chunk read 0, and their products are masked)
   const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)a.q, 0, a.nq * (NH * D * 2), 0x00020000);
-  const int row0 = lane / 8;  // of piece `lane`; piece lane + 64 c: row0 + 8 c, two queries on
-  const int qo = ((row0 >> 2) * NH + g * GQA + (row0 & 3)) * (D * 2) + 16 * ((lane & 7) ^ row0);
+      (void*)a.q, 0, a.nq * kChainQRow, 0x00020000);
   const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(a.ml + (size_t)(t0 >> 6) * (a.nq * NH)), 0, a.nq * (NH * 8), 0x00020000);
-  const int mo = (r * NH + g * GQA + h) * 8;
+      (void*)(a.ml + (size_t)(t0 >> 6) * (a.nq * NH)), 0, a.nq * kChainMRow, 0x00020000);
+  static_assert(kChainQRow == NH * D * 2 && kChainMRow == NH * (int)sizeof(f32x2) && GQA == 4, "");
   auto fetch = [&](int n, f32x2& mw) __attribute__((always_inline)) {
-    mw = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rm, mo, n * kR * (NH * 8), 0));
+    const ChainOff mo = chain_m_off(kR, n, r, g, h);
+    mw = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rm, mo.lane, mo.scalar, 0));
 #pragma unroll
-    for (int c = 0; c < kLd; c++)
+    for (int c = 0; c < kLd; c++) {
+      const ChainOff qo = chain_q_off(kR, n, c, lane, g);
       if (kPc >= 64 || lane < kPc)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (lds_void_t*)(lds + ((n & 1) * NKV + g) * kQB + 1024 * c), 16, qo,
-                                                 (n * kR + 2 * c) * (NH * D * 2), 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (lds_void_t*)(lds + ((n & 1) * NKV + g) * kQB + 1024 * c), 16,
+                                                 qo.lane, qo.scalar, 0, 0);
+    }
   };
   // (two steps' (m_b, w_b) in registers of their own: a copy from one to the
   // other would wait for the load)
