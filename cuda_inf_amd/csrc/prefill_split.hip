@@ -20,7 +20,8 @@
 //   S^T      = K Q^T (v_mfma_f32_16x16x32_f16): A = 16 keys x 16 dims per
 //            lane group as one 16-byte LDS read, fp8 -> fp16 exactly;
 //   softmax  in registers, as in prefill_tile.h (the running max moves only
-//            when a numerator would overflow fp16);
+//            when a numerator would overflow fp16); over H2O slots each tile
+//            against its own max (slot_exp);
 //   O^T     += vs (V^T P^T): V^T by ds_read_b64_tr_b8, the keys of a lane
 //            group's 8 elements being those its P holds; the group's V scale
 //            multiplies the tile's fp32 product, so V enters exactly.
@@ -48,6 +49,37 @@ struct SlotArgs {
   const int32_t* slot_pos;
   int n_live;
 };
+
+// Numerators of one 16-query tile over 64 slots, relative to the tile's own max
+// of each query: fp16 rounds the largest not at all and none of weight into
+// its subnormals, wherever in the buffer the largest score lies.  (Relative to
+// a running max, as over cached keys, 1024 queries over their own slots were
+// 3.18e-4 off 64 bits in place of 3.14e-4, and a buffer whose output is carried
+// by many slots 18 bits below the largest score 0.8 % off.)  S holds scores in
+// log2 units, -inf where masked.  Returns f = 2^(tile max - m), by which the
+// tile's products and sum enter O and l in fp32; m, the reference of O and l,
+// moves where f would pass 2^64.
+__device__ __forceinline__ float slot_exp(const f32x4 (&S)[4], float& m, float& l, f32x4 (&O)[4],
+                                          f16x8 (&P)[2]) {
+  float cm = -1e30f;  // (all masked: numerators 0)
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) cm = __builtin_fmaxf(cm, S[k][i]);
+  const float mt = pf_colmax(cm);
+  if (__any(mt > m + 64.f)) {
+    const float mn = mt > m + 64.f ? mt : m, corr = __builtin_amdgcn_exp2f(m - mn);
+    m = mn;
+    l *= corr;
+#pragma unroll
+    for (int d = 0; d < 4; d++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) O[d][i] *= corr;
+  }
+  const float rs = pf_exp<false>(S, 1.0f, mt, 0, 0, P), f = __builtin_amdgcn_exp2f(mt - m);
+  l = __builtin_fmaf(rs, f, l);
+  return f;
+}
 
 constexpr int kPsORow = 68;  // floats between two queries of a wave's partial O
 // bytes of a wave's LDS: the K and V tiles (and 64 slots' K scales, positions
@@ -145,7 +177,8 @@ __global__ __launch_bounds__(64 * kW) void k_prefill_split(PrefillArgs a, SlotAr
   const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // one tile: scores of the K operands kop(k) (16 keys each), softmax, pv(P)
-  auto attend = [&](int j, float c, bool first, auto kop, auto pv)
+  // with the factors of their products, vs over cached keys
+  auto attend = [&](int j, float c, float vs, bool first, auto kop, auto pv)
       __attribute__((always_inline)) {
     f32x4 S[kQT][4];
 #pragma unroll
@@ -180,6 +213,13 @@ __global__ __launch_bounds__(64 * kW) void k_prefill_split(PrefillArgs a, SlotAr
             S[t][k][i] = 64 * j + 16 * k + 4 * b + i > qmin + 16 * t + n ? -__builtin_inff() : S[t][k][i];
     }
     f16x8 P[kQT][2];
+    if constexpr (kSlots) {
+      float f[kQT];
+#pragma unroll
+      for (int t = 0; t < kQT; t++) f[t] = slot_exp(S[t], m[t], lsum[t], O[t], P[t]);
+      pv(P, f);
+      return;
+    }
 #pragma unroll
     for (int t = 0; t < kQT; t++) {
       float rs = first ? __builtin_inff() : pf_exp<false>(S[t], c, m[t], 0, 0, P[t]);
@@ -187,7 +227,10 @@ __global__ __launch_bounds__(64 * kW) void k_prefill_split(PrefillArgs a, SlotAr
         rs = pf_remax<false>(S[t], c, first, m[t], lsum[t], O[t], 0, 0, P[t]);
       lsum[t] += rs;
     }
-    pv(P);
+    float f[kQT];
+#pragma unroll
+    for (int t = 0; t < kQT; t++) f[t] = vs;
+    pv(P, f);
   };
   int first = 1;
   asm("" : "+s"(first));  // (opaque: the loop's first pass is not peeled into code of its own)
@@ -215,7 +258,7 @@ __global__ __launch_bounds__(64 * kW) void k_prefill_split(PrefillArgs a, SlotAr
       k0 = pf_cvt8(kk[0], kk[1]);
       k1 = pf_cvt8(kk[2], kk[3]);
     };
-    auto pv = [&](const f16x8 (&P)[kQT][2]) __attribute__((always_inline)) {
+    auto pv = [&](const f16x8 (&P)[kQT][2], const float (&f)[kQT]) __attribute__((always_inline)) {
       f16x8 sc[2];
       if constexpr (kSlots)
 #pragma unroll
@@ -235,19 +278,14 @@ __global__ __launch_bounds__(64 * kW) void k_prefill_split(PrefillArgs a, SlotAr
         }
 #pragma unroll
         for (int t = 0; t < kQT; t++) {
-          if constexpr (kSlots) {
-            O[t][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vop[0], P[t][0], O[t][d], 0, 0, 0);
-            O[t][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vop[1], P[t][1], O[t][d], 0, 0, 0);
-            continue;
-          }
           f32x4 T = __builtin_amdgcn_mfma_f32_16x16x32_f16(vop[0], P[t][0], zero, 0, 0, 0);
           T = __builtin_amdgcn_mfma_f32_16x16x32_f16(vop[1], P[t][1], T, 0, 0, 0);
 #pragma unroll
-          for (int i = 0; i < 4; i++) O[t][d][i] = __builtin_fmaf(T[i], vs, O[t][d][i]);
+          for (int i = 0; i < 4; i++) O[t][d][i] = __builtin_fmaf(T[i], f[t], O[t][d][i]);
         }
       }
     };
-    attend(j, c, first != 0, kop, pv);
+    attend(j, c, vs, first != 0, kop, pv);
     first = 0;
   }
   if (!kSlots && ntile > nfp8 && nfp8 % kW == w) {
@@ -267,7 +305,7 @@ __global__ __launch_bounds__(64 * kW) void k_prefill_split(PrefillArgs a, SlotAr
       *(u32x4*)(kt + r * 128 + 16 * (l & 7)) = v;
     }
     const _Float16* v16 = (const _Float16*)kt;
-    auto pv = [&](const f16x8 (&P)[kQT][2]) __attribute__((always_inline)) {
+    auto pv = [&](const f16x8 (&P)[kQT][2], const float (&)[kQT]) __attribute__((always_inline)) {
 #pragma unroll
       for (int d = 0; d < 4; d++)
 #pragma unroll
@@ -281,7 +319,7 @@ __global__ __launch_bounds__(64 * kW) void k_prefill_split(PrefillArgs a, SlotAr
             O[t][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vop, P[t][u], O[t][d], 0, 0, 0);
         }
     };
-    attend(nfp8, __builtin_fmaxf(a.qscale, 1e-30f), first != 0, kop, pv);
+    attend(nfp8, __builtin_fmaxf(a.qscale, 1e-30f), 1.0f, first != 0, kop, pv);
   }
 
   // ---- the wave's partial (its own LDS: the tiles are read): O[query][dim],

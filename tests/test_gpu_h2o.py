@@ -328,3 +328,33 @@ def test_attention_h2o_many_queries(orc, cia, dev, n_live, S, past, seed):
     inside a workgroup and a block, queries that end inside a step, more
     queries than the scratch holds at once (1048), the last S of the pair."""
     test_attention_h2o_kernel(orc, cia, dev, n_live, S, past, seed)
+
+
+@pytest.mark.parametrize("S", [15, 16, 200])
+def test_h2o_outputs_keep_small_numerators(cia, dev, S):
+    """Many slots far below the largest score, which carry the output: the first
+    slot of each of the first 16 blocks scores 18.5 ln 2 with V = 0, every other
+    slot 0 with V = 1600, so a query's output is 1600 w / (16 + w), w = (n - 16)
+    2^-18.5 (about 4.4).  Numerators rounded to fp16 relative to the largest
+    score would be 45 of 45.25 subnormal steps, 0.55 % or 2.4e-2 off; relative
+    to their own block, or with head room, each is within 2^-11."""
+    from cuda_inf_amd import kernels as K
+    n = 16384
+    kf = torch.zeros((n, 8, 64), dtype=torch.uint8, device=dev)
+    vf = torch.full((n, 8, 64), 0x38, dtype=torch.uint8, device=dev)  # 1.0
+    top = torch.arange(16, device=dev) * 64
+    kf[top, :, 0] = 0x38
+    vf[top] = 0
+    ks = torch.full((n, 8), 18.5 * np.log(2.0), dtype=torch.float16, device=dev)
+    vs = torch.full((n, 8), 1600.0, dtype=torch.float16, device=dev)
+    q = torch.zeros((S, 32, 64), dtype=torch.float16, device=dev)
+    q[:, :, 0] = 1.0
+    out = torch.empty_like(q)
+    mass = torch.zeros(n, device=dev)
+    ws = torch.empty(K.h2o_workspace_bytes(S, n), dtype=torch.uint8, device=dev)
+    print(f"h2o small numerators S={S}", flush=True)
+    K.attention_h2o(q, kf, vf, ks, vs, torch.arange(n, dtype=torch.int32, device=dev), n, out, mass,
+                    S, n, 1.0, ws)
+    torch.cuda.synchronize()
+    w = (n - 16) * np.exp(-float(ks[0, 0]))
+    assert_close_f16(_u16(out), np.full((S, 32, 64), 1600.0 * w / (16.0 + w)))
