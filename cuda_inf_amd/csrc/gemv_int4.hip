@@ -46,6 +46,8 @@ constexpr int kGemvWaves = 8;
 // us, M = 3 5.0 / 3.9, M = 16 10.1 / 3.9.)
 constexpr int kKsMinM = 3;
 constexpr int kKsMaxK = 4096;  // (its LDS scale table's groups)
+// Rows of x below which its sums take four chains a pass (k_gemm_int4_ks)
+constexpr int kChainsM = 56;
 // Beyond that K, rows of x from which the tile GEMM runs instead of the GEMV
 // (measured crossover)
 constexpr int kGemmMinM = 56;
@@ -636,17 +638,21 @@ __global__ __launch_bounds__(64 * kGemmWaves) void k_gemm_int4_big(GemvArgs a) {
 //   The scales of the tile's columns are fetched once, group-fastest as they
 //   lie in memory, into an LDS table.
 // As in the tile kernel, a group's products accumulate from zero and are added
-// in fp32 with the column's scale, in the order of the groups: the 8 waves'
-// products of a pass of 8 groups meet in LDS unscaled.  So an output has the
-// tile kernel's bits, whatever the shape -- a q/k/v sum in another order may
-// round to another fp16 value and that one to another E4M3 code in the cache.
+// in fp32 with the column's scale: the 8 waves' products of a pass of 8 groups
+// meet in LDS unscaled.  From kChainsM rows on they are added in the order of
+// the groups, so that an output has the tile kernel's bits, whatever the shape
+// -- a q/k/v sum in another order may round to another fp16 value and that one
+// to another E4M3 code in the cache.  Fewer rows, which the GEMV would take,
+// are added in four chains a pass: the GEMV's sums are trees, and 16 roundings
+// in a row are further off (out_proj into the residual, 2-norm from 64 bits:
+// GEMV 7.2e-8, in order 7.65e-8, so 6.3e-8).
 // (Two passes at K = 2048.  out_proj of 300 rows, a call: 14.7 us with one
 // meeting of the waves' own scaled sums and all four k steps' x in registers,
 // 11.8 as here.)
 constexpr int kKsWaves = 8;
 
 // grid = (ceil(rows / (16 kNT)), ceil(M / (16 kMT))), block = 512; K <= kKsMaxK
-template <int kOut, int kMT, int kNT>
+template <int kOut, int kMT, int kNT, bool kChains>
 __global__ __launch_bounds__(64 * kKsWaves) void k_gemm_int4_ks(GemvArgs a) {
   static_assert(kNT <= 4, "a wave's partial tile takes its x slot's place");
   __shared__ __attribute__((aligned(16))) uint8_t xs[kKsWaves * kMT * 4096];
@@ -755,7 +761,8 @@ __global__ __launch_bounds__(64 * kKsWaves) void k_gemm_int4_ks(GemvArgs a) {
   for (int u = 0; u < kPer; u++) v[u] = f32x4{0.f, 0.f, 0.f, 0.f};
   f32x4* part = (f32x4*)xs;  // [wave, 256 kMT apart][tile][lane] of 4 rows x 1 column
   // a pass's products meet: the tiles this wave adds up take its groups, from
-  // g0, in order; lane holds rows 4q .. 4q + 3 of column n16
+  // g0, in order (kChains: in four chains); lane holds rows 4q .. 4q + 3 of
+  // column n16
   auto meet = [&](int g0, const f32x4 (&Pg)[kMT][kNT]) __attribute__((always_inline)) {
     if (g0 + w < ng)
 #pragma unroll
@@ -766,6 +773,20 @@ __global__ __launch_bounds__(64 * kKsWaves) void k_gemm_int4_ks(GemvArgs a) {
 #pragma unroll
     for (int u = 0; u < kPer; u++) {
       const int t = w + kKsWaves * u < kTiles ? w + kKsWaves * u : 0;
+      if constexpr (kChains) {
+        f32x4 c[4] = {};
+#pragma unroll
+        for (int k = 0; k < kKsWaves; k++) {
+          if (g0 + k >= ng) break;
+          const f32x4 pv = part[k * kMT * 256 + t * 64 + l];
+          const float sc = ssc[g0 + k][16 * (t % kNT) + n16];
+#pragma unroll
+          for (int e = 0; e < 4; e++) c[k & 3][e] = __builtin_fmaf(pv[e], sc, c[k & 3][e]);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[u][e] += (c[0][e] + c[1][e]) + (c[2][e] + c[3][e]);
+        continue;
+      }
 #pragma unroll
       for (int k = 0; k < kKsWaves; k++) {
         if (g0 + k >= ng) break;
@@ -825,10 +846,12 @@ __global__ __launch_bounds__(64 * kKsWaves) void k_gemm_int4_ks(GemvArgs a) {
 
 template <int kOut, int kMT, int kNT>
 static void ks_launch(const GemvArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL((k_gemm_int4_ks<kOut, kMT, kNT>),
-                     dim3((unsigned)((a.rows + 16 * kNT - 1) / (16 * kNT)),
-                          (unsigned)((a.M + 16 * kMT - 1) / (16 * kMT))),
-                     dim3(64 * kKsWaves), 0, s, a);
+  const dim3 grid((unsigned)((a.rows + 16 * kNT - 1) / (16 * kNT)),
+                  (unsigned)((a.M + 16 * kMT - 1) / (16 * kMT)));
+  if (a.M < kChainsM)
+    hipLaunchKernelGGL((k_gemm_int4_ks<kOut, kMT, kNT, true>), grid, dim3(64 * kKsWaves), 0, s, a);
+  else
+    hipLaunchKernelGGL((k_gemm_int4_ks<kOut, kMT, kNT, false>), grid, dim3(64 * kKsWaves), 0, s, a);
 }
 
 // The K-split kernel's tile shape: the one of least expected time, c (the time

@@ -185,3 +185,29 @@ def test_qkv_big_tiles_bits(orc, cia, dev, M, seed):
         KK.gemv_int4(x, *W[n], y, N, K, M)
         torch.cuda.synchronize()
         assert torch.equal(out[n].view(torch.int16), y.half().view(torch.int16)), n
+
+
+@pytest.mark.parametrize("M,seed", [(3, 50), (23, 51), (55, 52)])
+def test_few_rows_no_further_off_than_gemv(orc, cia, dev, M, seed):
+    """out_proj into the residual for the rows that the GEMV would take too: the
+    2-norm distance from 64 bits is no larger than that of the GEMV, which runs
+    for two rows at a time (its trees of sums have fewer roundings in a row than
+    a sum over the 16 groups in order)."""
+    from cuda_inf_amd import kernels as KK
+    rng = np.random.default_rng(seed)
+    N = K = 2048
+    packed, scales = _weights(rng, N, K, orc)
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    y0 = rng.standard_normal((M, N)).astype(np.float32)
+    nib = np.stack((packed & 15, packed >> 4), -1).reshape(N, K).astype(np.float64) - 8.0
+    w = nib * np.repeat(scales.view(np.float16).astype(np.float64), 128, axis=1)
+    ref = y0.astype(np.float64) + x.astype(np.float64) @ w.T
+    xd, pd, sd, y, z = _t(x, dev), _t(packed, dev), _t(scales, dev), _t(y0, dev), _t(y0, dev)
+    print(f"few rows M={M}", flush=True)
+    KK.gemv_int4(xd, pd, sd, y, N, K, M, add=True)
+    for r in range(0, M, 2):
+        n = min(2, M - r)
+        KK.gemv_int4(xd[r:r + n], pd, sd, z[r:r + n], N, K, n, add=True)
+    torch.cuda.synchronize()
+    err, gemv = (np.linalg.norm(t.cpu().numpy() - ref) / np.linalg.norm(ref) for t in (y, z))
+    assert err <= gemv, (err, gemv)
