@@ -692,10 +692,11 @@ __global__ __launch_bounds__(64 * kKsWaves) void k_gemm_int4_ks(GemvArgs a) {
   // the output tiles this wave adds up at the end (w, w + 8, ..): their
   // residual goes out with the operands
   constexpr int kTiles = kMT * kNT, kPer = (kTiles + kKsWaves - 1) / kKsWaves;
-  float yo[kPer][4];
+  float yo[kPer][4] = {};
 #pragma unroll
   for (int u = 0; u < kPer; u++) {
-    const int t = w + kKsWaves * u < kTiles ? w + kKsWaves * u : 0;
+    const int t = w + kKsWaves * u;
+    if (kOut != kOutAdd || t >= kTiles) break;
     const OutCol<kOut> o(a, r0 + 16 * (t % kNT) + n16);
 #pragma unroll
     for (int e = 0; e < 4; e++) {
