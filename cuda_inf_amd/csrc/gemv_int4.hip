@@ -21,6 +21,7 @@
 // output.  (Measured at 3072 and 2048 rows: one row per wave beats 2, 4 or
 // 8; the staged x beats per-wave x loads.)
 #include "common.h"
+#include "int4_shape.h"
 
 namespace cia {
 
@@ -41,21 +42,8 @@ struct GemvArgs {
 };
 
 constexpr int kGemvWaves = 8;
-// Rows of x from which the K-split matrix-core GEMM runs, for K up to
-// kKsMaxK.  (q/k/v of 2048, 512 and 512 rows, GEMV / K-split: M = 2 3.7 / 3.8
-// us, M = 3 5.0 / 3.9, M = 16 10.1 / 3.9.)
-constexpr int kKsMinM = 3;
-constexpr int kKsMaxK = 4096;  // (its LDS scale table's groups)
-// Rows of x below which its sums take four chains a pass (k_gemm_int4_ks)
+// Rows of x below which the K-split kernel's sums take four chains a pass
 constexpr int kChainsM = 56;
-// Beyond that K, rows of x from which the tile GEMM runs instead of the GEMV
-// (measured crossover)
-constexpr int kGemmMinM = 56;
-// Rows of x from which the tile GEMM runs for any K.  (q/k/v, K-split / tile:
-// M = 512 17.4 / 24.4 us, 768 26.1 / 24.9; out_proj 768 20.6 / 27.7, 1024
-// 25.5 / 28.8.  The line does not depend on the rows of W, so that one
-// matrix gives the same bits alone and in a q/k/v launch.)
-constexpr int kTileMinM = 769;
 
 // nibbles sh..sh+3 and sh+16..sh+19 of w as fp16 (nibble - 8), exact
 __device__ __forceinline__ f16x2 nib_pair(uint32_t w, int sh) {
@@ -465,7 +453,6 @@ __global__ __launch_bounds__(64 * kGemmWaves) void k_gemm_int4(GemvArgs a) {
 // (q/k/v of 4096 rows, kNT = 3, one round of 256 workgroups: 77 -> 58 us, 885
 // TFLOP/s; out_proj, kNT = 2: 66 -> 51.)
 constexpr int kBigRows = 256;
-constexpr int kBigMaxK = 2048;
 
 // grid = the tiles, ceil(rows / (64 kNT)) * ceil(M / 256), up to a multiple of 8;
 // block = 512
@@ -855,73 +842,28 @@ static void ks_launch(const GemvArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((k_gemm_int4_ks<kOut, kMT, kNT, false>), grid, dim3(64 * kKsWaves), 0, s, a);
 }
 
-// The K-split kernel's tile shape: the one of least expected time, c (the time
-// of one round of workgroups less the 2.2 us of an empty launch, measured) times
-// the rounds.  A 4-row-tile workgroup has a compute unit to itself (128 KB of
-// LDS), so its rounds are whole; the smaller ones overlap from one round into
-// the next.  (Launches of 2048 rows of W, in us, chosen shape first: M = 16:
-// 1x1 4.2, 2x2 5.7; 64: 1x2 5.1, 2x2 5.7, 1x1 5.7; 128: 2x2 6.0, 4x4 11.3,
-// 1x1 8.9; 300: 4x3 9.9, 2x2 11.5, 4x4 12.0, 1x1 16.9; 512: 4x4 13.4, 2x2
-// 14.0, 1x1 25.0.)
-struct KsShape {
-  int mt, nt;
-  float c;
-};
-constexpr KsShape kKsShapes[] = {{1, 1, 1.7f}, {1, 2, 2.5f}, {2, 2, 3.4f}, {2, 3, 4.4f},
-                                 {4, 3, 7.2f}, {4, 4, 9.3f}};
-
-static float ks_time(const KsShape& k, int M, int rows) {
-  const int wgs = ((rows + 16 * k.nt - 1) / (16 * k.nt)) * ((M + 16 * k.mt - 1) / (16 * k.mt));
-  const float r = (float)wgs / 256.0f;
-  return k.c * (r <= 1.0f ? 1.0f : (k.mt == 4 ? (float)((wgs + 255) / 256) : r));
+template <int kOut, int kNT>
+static void big_launch(const GemvArgs& a, long tiles, hipStream_t s) {
+  hipLaunchKernelGGL((k_gemm_int4_big<kOut, kNT>), dim3((unsigned)((tiles + 7) / 8 * 8)),
+                     dim3(64 * kGemmWaves), 0, s, a);
 }
 
 // the matrix-core kernels, by the launch's output form
-// Time of a tiling of many rows: rounds of 256 workgroups (one a compute unit)
-// times a tile's own time, 128 x 128 = 100.  (One round / two, K = 2048: 128 x
-// 128 29 / 51 us, 256 x 128 35 / 72, 256 x 192 46 to 58.  q/k/v of 1024 rows:
-// 128 x 128 29 us, the others 35 and 46; 2048 rows: 51, 39 and 51; 3000: 74,
-// 71 and 52.  out_proj of 2048 rows: 36, 46 and 61; 3000: 59, 48 and 62.)  The
-// sums are the same in each, so the choice may depend on the rows of W.
-static long tile_count(const GemvArgs& a, int cols, int xrows) {
-  return (a.rows + (long)cols - 1) / cols * ((a.M + (long)xrows - 1) / xrows);
-}
-static long big_time(const GemvArgs& a, int cols, int xrows, int cost) {
-  return (tile_count(a, cols, xrows) + 255) / 256 * cost;
-}
-
 template <int kOut>
 static void gemm_launch(const GemvArgs& a, hipStream_t s) {
-  if (a.M < kTileMinM && a.K <= kKsMaxK) {
-    int b = 0;
-    for (int i = 1; i < (int)(sizeof(kKsShapes) / sizeof(kKsShapes[0])); i++)
-      if (ks_time(kKsShapes[i], a.M, a.rows) < ks_time(kKsShapes[b], a.M, a.rows)) b = i;
-    switch (10 * kKsShapes[b].mt + kKsShapes[b].nt) {
-      case 11: return ks_launch<kOut, 1, 1>(a, s);
-      case 12: return ks_launch<kOut, 1, 2>(a, s);
-      case 22: return ks_launch<kOut, 2, 2>(a, s);
-      case 23: return ks_launch<kOut, 2, 3>(a, s);
-      case 43: return ks_launch<kOut, 4, 3>(a, s);
-      case 44: return ks_launch<kOut, 4, 4>(a, s);
-    }
-  }
-  const dim3 block(64 * kGemmWaves);
-  if (a.K <= kBigMaxK) {
-    const long t = big_time(a, kTile, kTile, 100), t2 = big_time(a, 128, kBigRows, 145),
-               t3 = big_time(a, 192, kBigRows, 200);
-    const int n2 = (int)(tile_count(a, 128, kBigRows) + 7) / 8 * 8,
-              n3 = (int)(tile_count(a, 192, kBigRows) + 7) / 8 * 8;
-    if (t2 < t && t2 <= t3) {
-      hipLaunchKernelGGL((k_gemm_int4_big<kOut, 2>), dim3(n2), block, 0, s, a);
-      return;
-    }
-    if (t3 < t) {
-      hipLaunchKernelGGL((k_gemm_int4_big<kOut, 3>), dim3(n3), block, 0, s, a);
-      return;
-    }
+  const Int4Shape& sh = kInt4Shapes[int4_shape(a.M, a.rows, a.K)];
+  switch (1000 * sh.xrows + sh.cols) {
+    case 16016: return ks_launch<kOut, 1, 1>(a, s);
+    case 16032: return ks_launch<kOut, 1, 2>(a, s);
+    case 32032: return ks_launch<kOut, 2, 2>(a, s);
+    case 32048: return ks_launch<kOut, 2, 3>(a, s);
+    case 64048: return ks_launch<kOut, 4, 3>(a, s);
+    case 64064: return ks_launch<kOut, 4, 4>(a, s);
+    case 256128: return big_launch<kOut, 2>(a, int4_tiles(sh, a.M, a.rows), s);
+    case 256192: return big_launch<kOut, 3>(a, int4_tiles(sh, a.M, a.rows), s);
   }
   hipLaunchKernelGGL(k_gemm_int4<kOut>, dim3((unsigned)((a.rows + kTile - 1) / kTile),
-                     (unsigned)((a.M + kTile - 1) / kTile)), block, 0, s, a);
+                     (unsigned)((a.M + kTile - 1) / kTile)), dim3(64 * kGemmWaves), 0, s, a);
 }
 
 template <int kM>
@@ -943,7 +885,7 @@ static void gemv_launch(const GemvArgs& a, hipStream_t s) {
 static int gemv_run(GemvArgs& a, void* stream) {
   a.rows = a.mat[0].N + a.mat[1].N + a.mat[2].N;
   hipStream_t s = (hipStream_t)stream;
-  if (a.M >= (a.K <= kKsMaxK ? kKsMinM : kGemmMinM)) {
+  if (!int4_gemv(a.M, a.rows, a.K, a.add)) {
     if (a.mat[0].y16)
       gemm_launch<kOutF16>(a, s);
     else if (a.add)

@@ -1,5 +1,7 @@
 """Shared fixtures: the `gpu` marker, library loading, tolerance helpers."""
 import os
+import shutil
+import subprocess
 import sys
 
 import numpy as np
@@ -56,3 +58,27 @@ def dev():
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
     return torch.device("cuda:0")
+
+
+@pytest.fixture(scope="session")
+def int4_choose(tmp_path_factory):
+    """(rows of x, rows of W, K) -> (index of the chosen kInt4Shapes, whether the
+    GEMV runs: sums stored, sums added), from cuda_inf_amd/csrc/int4_shape.h."""
+    if shutil.which("g++") is None:
+        pytest.skip("needs g++")
+    d = tmp_path_factory.mktemp("int4_shape")
+    src, exe = str(d / "choose.cpp"), str(d / "choose")
+    with open(src, "w") as f:
+        f.write('#include <cstdio>\n#include "int4_shape.h"\n'
+                "int main() { int m, r, k; while (std::scanf(\"%d %d %d\", &m, &r, &k) == 3)\n"
+                "  std::printf(\"%d %d %d\\n\", cia::int4_shape(m, r, k), cia::int4_gemv(m, r, k, false),\n"
+                "              cia::int4_gemv(m, r, k, true)); }\n")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", os.path.join(ROOT, "cuda_inf_amd", "csrc"),
+                    src, "-o", exe], check=True)
+
+    def run(sizes):
+        r = subprocess.run([exe], input="".join("%d %d %d\n" % s for s in sizes), text=True,
+                           capture_output=True, timeout=60, check=True)
+        return [tuple(map(int, l.split())) for l in r.stdout.splitlines()]
+
+    return run

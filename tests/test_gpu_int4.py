@@ -55,9 +55,28 @@ CASES = [
     (2048, 4096, 2, "normal", 5),
     (64, 2048, 1, "extreme", 6),
     (512, 2048, 9, "normal", 7),
-    (2048, 2048, 96, "normal", 8),   # matrix-core path from 56 rows of x
+    (2048, 2048, 96, "normal", 8),
     (100, 384, 200, "normal", 9),    # ragged tiles in both directions
     (520, 2048, 300, "extreme", 13),
+    # the K-split GEMM's edges: first M, one row past a tile, rows of W that end
+    # inside a tile, fewer groups than waves (K = 128, 384), a second and a
+    # partial third pass over the groups (K = 1152, 2176), the largest K
+    (100, 128, 3, "normal", 20),
+    (130, 384, 16, "normal", 21),
+    (47, 1152, 17, "normal", 22),
+    (200, 2176, 33, "normal", 23),
+    (48, 4096, 65, "normal", 24),
+    (2000, 256, 130, "normal", 26),
+    (2048, 128, 300, "normal", 27),
+    (2050, 384, 511, "normal", 28),
+    (33, 256, 768, "normal", 29),
+    # its multi-pass forms at wider tiles, and the tile GEMM beyond its K
+    (2048, 2176, 130, "normal", 31),
+    (2048, 4096, 300, "normal", 32),
+    (2048, 2176, 511, "normal", 33),
+    (48, 4224, 40, "normal", 25),    # (the GEMV: 55 rows and fewer)
+    (48, 4224, 60, "normal", 34),
+    (200, 4096, 2100, "normal", 30),
 ]
 
 
@@ -82,7 +101,8 @@ def test_gemv_int4(orc, cia, dev, N, K, M, kind, seed):
            extra=2 * np.finfo(np.float32).eps * (np.abs(y0) + np.abs(ref)))
 
 
-@pytest.mark.parametrize("M,seed", [(1, 10), (3, 11), (6, 12), (130, 14)])
+@pytest.mark.parametrize("M,seed", [(1, 10), (2, 31), (3, 11), (6, 12), (16, 32), (40, 33), (130, 14),
+                                    (300, 34), (600, 37)])
 def test_qkv_proj_int4(orc, cia, dev, M, seed):
     """q/k/v in one launch with the fp16 conversion fused: each output is
     the fp16 rounding of the same kernel's fp32 sum (compared with the fp32
@@ -112,34 +132,74 @@ def test_qkv_proj_int4(orc, cia, dev, M, seed):
                extra=np.abs(ref) * 2.0 ** -11 + 2.0 ** -25)
 
 
-# The K-split GEMM (3 to 768 rows of x, K up to 4096) at the edges of its
-# dispatch and tiles: first and last M, one row past a tile, rows of W that
-# end inside a tile, fewer groups than waves (K = 128, 384), a second and a
-# partial third pass over the groups (K = 1152, 2176), the largest K and the
-# first beyond it, and M on both sides of each shape's choice.
-KSPLIT = [(100, 128, 3, 20), (130, 384, 16, 21), (47, 1152, 17, 22), (200, 2176, 33, 23),
-          (48, 4096, 65, 24), (48, 4224, 40, 25), (2000, 256, 130, 26), (2048, 128, 300, 27),
-          (2050, 384, 511, 28), (33, 256, 768, 29), (33, 256, 769, 30)]
+# Every matrix-core kernel and tile shape adds a row's groups in the same order
+# from 56 rows of x on: launches over the first M rows, one M for each shape that
+# the rule of a size takes, have the bits of one launch of the 128 x 128 tiles.
+# (K above 2048: three and four passes of the K-split kernel, no 256-row tiles.)
+@pytest.mark.parametrize("N,K,shapes,seed", [
+    (64, 2048, {0, 1}, 60), (512, 2048, {0, 1, 2, 3, 4, 5}, 61), (2048, 2048, {1, 2, 3, 4, 5, 7}, 62),
+    (8192, 2048, {5, 2, 7, 8}, 63), (2050, 384, {2, 3, 4, 5, 7}, 64),
+    (2048, 2176, {1, 2, 3, 4, 5}, 65), (512, 4096, {0, 1, 2, 3, 4, 5}, 66)])
+def test_kernels_have_the_tile_kernels_bits(orc, cia, dev, int4_choose, N, K, shapes, seed):
+    from cuda_inf_amd import kernels as KK
+    rng = np.random.default_rng(seed)
+    rows = np.arange(56, 2400)
+    chosen = np.array([c[0] for c in int4_choose([(int(m), N, K) for m in rows])])
+    first = {}  # shape -> a ragged M that takes it, its first one and its last
+    for i in sorted(set(chosen)):
+        at = rows[chosen == i]
+        first[i] = sorted({int(at[0]), int(at[len(at) // 2]) | 1, int(at[-1])} & set(at.tolist()))
+    assert shapes <= set(first) - {6}
+    M, most = first[6][-1], max(m for ms in first.values() for m in ms)
+    packed, scales = _weights(rng, N, K, orc)
+    x = rng.standard_normal((most, K)).astype(np.float16)
+    xd, pd, sd = _t(x, dev), _t(packed, dev), _t(scales, dev)
+    for add in (False, True):
+        y0 = torch.full((most, N), 0.5 if add else float("nan"), dtype=torch.float32, device=dev)
+        y = y0[:M].clone()
+        KK.gemv_int4(xd[:M], pd, sd, y, N, K, M, add=add)
+        for i, ms in first.items():
+            for m in ms:
+                z = y0[:m].clone()
+                print(f"N={N} K={K} shape {i} M={m} add={add}", flush=True)
+                KK.gemv_int4(xd[:m], pd, sd, z, N, K, m, add=add)
+                torch.cuda.synchronize()
+                n = min(m, M)
+                assert torch.equal(z[:n], y[:n]) and not z.isnan().any(), (i, m)
 
 
-@pytest.mark.parametrize("N,K,M,seed", KSPLIT)
-def test_gemm_ksplit(orc, cia, dev, N, K, M, seed):
-    test_gemv_int4(orc, cia, dev, N, K, M, "normal", seed)
+@pytest.mark.parametrize("N,K,seed", [(64, 2048, 70), (3072, 2048, 71), (8192, 2176, 72)])
+def test_few_rows_have_the_same_bits(orc, cia, dev, int4_choose, N, K, seed):
+    """Below 56 rows of x the sums take another order (four chains a pass), the
+    same in every tile shape: 55 rows against slices of them."""
+    from cuda_inf_amd import kernels as KK
+    rng = np.random.default_rng(seed)
+    M, lo = 55, 3 + 2 * int4_choose([(3, N, K)])[0][1]
+    packed, scales = _weights(rng, N, K, orc)
+    xd = _t(rng.standard_normal((M, K)).astype(np.float16), dev)
+    pd, sd = _t(packed, dev), _t(scales, dev)
+    y = torch.zeros((M, N), dtype=torch.float32, device=dev)
+    KK.gemv_int4(xd, pd, sd, y, N, K, M)
+    for m in (lo, 16, 17, 33, 40):
+        z = torch.zeros((m, N), dtype=torch.float32, device=dev)
+        print(f"N={N} K={K} M={m}", flush=True)
+        KK.gemv_int4(xd[:m], pd, sd, z, N, K, m)
+        torch.cuda.synchronize()
+        assert torch.equal(z, y[:m]), m
 
 
-# The 256-row tiles (more than 768 rows of x, K up to 2048, where they need
-# fewer rounds of 256 workgroups): 128 and 192 columns a tile, each with ragged
-# last rows and columns and tiles past the end of the grid; one, two, three and
-# sixteen groups.  Their sums are in the 128 x 128 tiles' order, so the rows
-# have the bits of launches over slices of them that take those; the first and
-# last rows are checked against the oracle.
+# The 256-row tiles: 128 and 192 columns a tile, each with ragged last rows and
+# columns and tiles past the end of the grid; one, two, three and sixteen groups.
+# The rows have the bits of launches over slices of them, whatever those take;
+# the first and last rows are checked against the oracle.
 BIG_TILES = [(2080, 128, 2060, 2, 40), (2080, 384, 2060, 2, 41), (4100, 256, 2561, 3, 42),
              (1100, 2048, 4000, 4, 43), (3072, 2048, 2700, 3, 44)]
 
 
 @pytest.mark.parametrize("N,K,M,parts,seed", BIG_TILES)
-def test_gemm_big_tiles(orc, cia, dev, N, K, M, parts, seed):
+def test_gemm_big_tiles(orc, cia, dev, int4_choose, N, K, M, parts, seed):
     from cuda_inf_amd import kernels as KK
+    assert int4_choose([(M, N, K)])[0][0] >= 7
     rng = np.random.default_rng(seed)
     packed, scales = _weights(rng, N, K, orc, "normal")
     x = rng.standard_normal((M, K)).astype(np.float16)
@@ -151,7 +211,6 @@ def test_gemm_big_tiles(orc, cia, dev, N, K, M, parts, seed):
         KK.gemv_int4(xd, pd, sd, y, N, K, M, add=add)
         for r in torch.arange(M).tensor_split(parts):
             r0, n = int(r[0]), len(r)
-            assert n > 768
             KK.gemv_int4(xd[r0:r0 + n], pd, sd, z[r0:r0 + n], N, K, n, add=add)
         torch.cuda.synchronize()
         assert torch.equal(y, z)
@@ -159,13 +218,6 @@ def test_gemm_big_tiles(orc, cia, dev, N, K, M, parts, seed):
             ends = np.r_[0:3, M - 3:M]
             ref, ab = orc.gemv_int4(x[ends], packed, scales, want_absum=True)
             _check(y.cpu().numpy()[ends], ref, ab, "y")
-
-
-@pytest.mark.parametrize("M,seed", [(2, 31), (16, 32), (40, 33), (300, 34)])
-def test_qkv_shapes_bits(orc, cia, dev, M, seed):
-    """q/k/v in one launch have the bits of the three matrices alone,
-    whatever tile shapes the launches take."""
-    test_qkv_proj_int4(orc, cia, dev, M, seed)
 
 
 @pytest.mark.parametrize("M,seed", [(1600, 35), (2700, 36)])
@@ -187,7 +239,7 @@ def test_qkv_big_tiles_bits(orc, cia, dev, M, seed):
         assert torch.equal(out[n].view(torch.int16), y.half().view(torch.int16)), n
 
 
-@pytest.mark.parametrize("M,seed", [(3, 50), (23, 51), (55, 52)])
+@pytest.mark.parametrize("M,seed", [(3, 50), (5, 53), (23, 51), (55, 52)])
 def test_few_rows_no_further_off_than_gemv(orc, cia, dev, M, seed):
     """out_proj into the residual for the rows that the GEMV would take too: the
     2-norm distance from 64 bits is no larger than that of the GEMV, which runs
