@@ -42,9 +42,6 @@ struct GemvArgs {
 };
 
 constexpr int kGemvWaves = 8;
-// Rows of x below which the K-split kernel's sums take four chains a pass
-constexpr int kChainsM = 56;
-
 // nibbles sh..sh+3 and sh+16..sh+19 of w as fp16 (nibble - 8), exact
 __device__ __forceinline__ f16x2 nib_pair(uint32_t w, int sh) {
   const uint32_t v = ((w >> sh) & 0x000F000Fu) | 0x64006400u;  // 1024 + nibble

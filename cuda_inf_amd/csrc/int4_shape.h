@@ -1,13 +1,17 @@
 // int4_shape.h -- which matrix-core kernel and tile an INT4 projection launch
-// takes (gemv_int4.hip).  All of them give a row the same bits from 56 rows of
-// x on, so the choice is by time alone and may depend on the rows of W.  Plain
-// C++, so that the rule is checked against measured times on the CPU.
+// takes (gemv_int4.hip).  All of them give a row the same bits from kChainsM rows
+// of x on, and the K-split kernel's shapes do below, so the choice is by time
+// alone and may depend on the rows of W.  Plain C++, so that the rule is checked
+// against measured times on the CPU.
 #pragma once
 
 namespace cia {
 
 constexpr int kKsMaxK = 4096;   // K-split kernel: its LDS scale table's groups
 constexpr int kBigMaxK = 2048;  // 256-row tiles: the LDS
+// Rows of x below which the K-split kernel's sums take four chains a pass, an
+// order of its own: no other matrix-core kernel runs there
+constexpr int kChainsM = 56;
 // The largest number of rows whose x the K-split shapes were measured with
 constexpr int kKsMaxM = 2048;
 
@@ -55,6 +59,7 @@ constexpr int int4_shape(int M, int rows, int K) {
     const Int4Shape& s = kInt4Shapes[i];
     if (s.kernel == kInt4Ks && (K > kKsMaxK || M > kKsMaxM)) continue;
     if (s.kernel == kInt4Big && K > kBigMaxK) continue;
+    if (s.kernel != kInt4Ks && K <= kKsMaxK && M < kChainsM) continue;
     const float ti = int4_time(s, M, rows, K);
     if (best < 0 || ti < t) {
       best = i;
@@ -75,7 +80,7 @@ constexpr int int4_shape(int M, int rows, int K) {
 // in a q/k/v launch, and the two kernels add in different orders.
 constexpr bool int4_gemv(int M, int rows, int K, bool add) {
   if (M <= 2) return true;
-  if (M >= 56) return false;
+  if (M >= kChainsM) return false;
   if (K > kKsMaxK) return true;
   if (add) return K > 1536 && ((long)rows + 7) / 8 * ((M + 3) / 4) <= 256;
   return K > 2048 && M < 5;
