@@ -236,9 +236,11 @@ __global__ __launch_bounds__(64 * kW) void k_prefill_split(PrefillArgs a, SlotAr
   asm("" : "+s"(first));  // (opaque: the loop's first pass is not peeled into code of its own)
   for (int j = w; j < nf; j += kW) {
     float c = 1.0f, vs = 1.0f;
-    bool seen = true;  // by some query of the workgroup
+    bool seen = true;   // by some query of the workgroup
+    bool kinf = false;  // a slot's K scale is infinite
     if constexpr (kSlots) {
       seen = __any(cur.pos <= qlast);
+      kinf = __any((cur.ks & 0x7FFF) == 0x7C00);
       lks[l] = h2f(cur.ks) * a.qscale;
       lpos[l] = cur.pos;
       lvs[l] = __builtin_bit_cast(_Float16, cur.vs);
@@ -257,6 +259,14 @@ __global__ __launch_bounds__(64 * kW) void k_prefill_split(PrefillArgs a, SlotAr
       const u32x4 kk = *(const u32x4*)(kt + (k & 1 ? ko1 : ko0) + 1024 * k);
       k0 = pf_cvt8(kk[0], kk[1]);
       k1 = pf_cvt8(kk[2], kk[3]);
+      if constexpr (kSlots)
+        if (kinf) {
+          // its values are infinite or 0 * inf before the product, which is
+          // then NaN unless every term has one sign
+          const _Float16 x = __builtin_isinf(lks[16 * k + n]) ? (_Float16)__builtin_inff() : (_Float16)1.0f;
+          k0 *= x;
+          k1 *= x;
+        }
     };
     auto pv = [&](const f16x8 (&P)[kQT][2], const float (&f)[kQT]) __attribute__((always_inline)) {
       f16x8 sc[2];

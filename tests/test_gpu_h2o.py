@@ -322,11 +322,13 @@ def test_h2o_layers_sharing_ws_mass(cia, dev):
 
 @pytest.mark.parametrize("n_live,S,past,seed", [
     (3, 16, 0, 40), (64, 33, 10, 41), (1030, 17, 900, 42), (2500, 16, 3000, 43),
-    (70, 1100, 30, 44), (1024, 15, 600, 45), (257, 130, 200, 46)])
+    (70, 1100, 30, 44), (1024, 15, 600, 45), (257, 130, 200, 46),
+    (700, 40, 650, 47), (1800, 200, 1700, 48), (3000, 150, 2900, 49)])
 def test_attention_h2o_many_queries(orc, cia, dev, n_live, S, past, seed):
     """The many-query launches: each slots-per-workgroup choice, slots that end
     inside a workgroup and a block, queries that end inside a step, more
-    queries than the scratch holds at once (1048), the last S of the pair."""
+    queries than the scratch holds at once (1048), the last S of the pair; of the
+    output launch, 16 queries by 4, 8 and 16 waves and 32 queries by 4 and 8."""
     test_attention_h2o_kernel(orc, cia, dev, n_live, S, past, seed)
 
 
@@ -337,7 +339,7 @@ def test_h2o_outputs_keep_small_numerators(cia, dev, S):
     slot 0 with V = 1600, so a query's output is 1600 w / (16 + w), w = (n - 16)
     2^-18.5 (about 4.4).  Numerators rounded to fp16 relative to the largest
     score would be 45 of 45.25 subnormal steps, 0.55 % or 2.4e-2 off; relative
-    to their own block, or with head room, each is within 2^-11."""
+    to their own block each is within 2^-11."""
     from cuda_inf_amd import kernels as K
     n = 16384
     kf = torch.zeros((n, 8, 64), dtype=torch.uint8, device=dev)
@@ -358,3 +360,64 @@ def test_h2o_outputs_keep_small_numerators(cia, dev, S):
     torch.cuda.synchronize()
     w = (n - 16) * np.exp(-float(ks[0, 0]))
     assert_close_f16(_u16(out), np.full((S, 32, 64), 1600.0 * w / (16.0 + w)))
+
+
+NONFINITE = ["k_nan", "k_inf", "v_nan", "v_inf", "k_scale_inf", "v_scale_inf", "none_seen", "minus_inf"]
+
+
+@pytest.mark.parametrize("S", [15, 16, 150])
+@pytest.mark.parametrize("kind", NONFINITE)
+def test_attention_h2o_nonfinite(orc, cia, dev, S, kind):
+    """Values that are no numbers, through the launch pair (15 queries) and the
+    many-query launches: a slot whose K or V is NaN or infinite as it was
+    quantised (kv head 2), or whose scale alone is infinite, queries that see no
+    slot, and a slot that scores -inf.  Outputs are NaN and infinite where the
+    oracle's are and close elsewhere; masses are NaN where the oracle's are and
+    have its bits elsewhere."""
+    from cuda_inf_amd import kernels as K
+    n, past = 1500, 2000
+    rng = np.random.default_rng(S)
+    k, v = (rng.standard_normal((n, 8, 64)).astype(np.float16) for _ in range(2))
+    q = rng.standard_normal((S, 32, 64)).astype(np.float16)
+    t, d = 700, 5
+    if kind[0] in "kv" and "scale" not in kind:
+        (k if kind[0] == "k" else v)[t, 2, d] = np.nan if kind.endswith("nan") else np.inf
+    if kind == "minus_inf":  # every product of kv head 2's slot is -inf or less than 0
+        q[:, 8:12] = np.abs(q[:, 8:12]) + np.float16(0.1)
+        k[t, 2] = -np.abs(k[t, 2]) - np.float16(0.1)
+    kf = torch.zeros((n, 8, 64), dtype=torch.uint8, device=dev)
+    vf = torch.zeros_like(kf)
+    ks = torch.zeros((n, 8), dtype=torch.float16, device=dev)
+    vs = torch.zeros_like(ks)
+    dst = torch.arange(n, dtype=torch.int32, device=dev)
+    K.kv_quant_write(torch.from_numpy(k).to(dev), torch.from_numpy(v).to(dev), kf, vf, ks, vs, dst, n)
+    if kind in ("k_scale_inf", "minus_inf"):
+        ks[t, 2] = float("inf")
+    if kind == "v_scale_inf":
+        vs[t, 2] = float("inf")
+    pos = rng.permutation(n).astype(np.int32)
+    if kind == "none_seen":
+        pos = past + 5 + pos % 7  # queries 0..4 see nothing, 5..11 a part
+    attn0 = np.abs(rng.standard_normal(n)).astype(np.float32)
+    r_attn = attn0.copy()
+    with np.errstate(invalid="ignore"):
+        _, r32 = orc.attention_h2o(_u16(torch.from_numpy(q)), kf.cpu().numpy(), vf.cpu().numpy(), _u16(ks),
+                                   _u16(vs), pos, n, r_attn, S, past)
+    out = torch.zeros((S, 32, 64), dtype=torch.float16, device=dev)
+    mass = torch.from_numpy(attn0.copy()).to(dev)
+    ws = torch.zeros(K.h2o_workspace_bytes(S, n), dtype=torch.uint8, device=dev)
+    print(f"h2o non-finite {kind} S={S}", flush=True)
+    K.attention_h2o(torch.from_numpy(q).to(dev), kf, vf, ks, vs, torch.from_numpy(pos).to(dev), n, out,
+                    mass, S, past, 0.125, ws)
+    torch.cuda.synchronize()
+    got, gm = out.float().cpu().numpy(), mass.cpu().numpy()
+    assert np.array_equal(np.isnan(gm), np.isnan(r_attn))
+    fin = ~np.isnan(gm)
+    assert np.array_equal(gm[fin].view(np.uint32), r_attn[fin].view(np.uint32))
+    assert np.array_equal(np.isnan(got), np.isnan(r32)), (np.isnan(got).sum(), np.isnan(r32).sum())
+    inf = np.isinf(r32)
+    assert np.array_equal(got[inf], r32[inf])
+    fin = np.isfinite(r32)
+    assert_close_f16(got[fin], r32[fin], what=kind)
+    if kind == "none_seen":
+        assert np.isnan(got[:5]).all() and np.isfinite(got[5:]).all()
