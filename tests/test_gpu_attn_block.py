@@ -117,3 +117,34 @@ def test_attn_block_loop_matches_single_calls(orc, cia, dev):
     assert [L.committed for L in layers[0]] == [L.committed for L in layers[1]] == [128] * nl
     assert torch.equal(h_a, h_b)
     assert torch.isfinite(h_a).all()
+
+
+def test_short_turn_cache_beside_single_tokens(orc, cia, dev):
+    """The cache bytes of 64 tokens given as turns of 40 and 24 beside those of
+    the same tokens given one by one.  Projections of 3 to 55 rows add their
+    products in another order than those of one row, so an fp16 k or v may round
+    to its neighbour: sums some 1e-7 of their size apart cross a rounding
+    boundary of 2^-11 in about 1e-3 of the values.  Of those, 2^-7 sit at an E4M3
+    boundary, seven bits coarser, and a head's largest value (one in 4096) takes
+    the group's scale with it, by 2^-10 at most, which moves 2^-7 of its codes.
+    Expected share of codes that differ: 1e-3 (2^-7 + 2^-7) = 1.6e-5; the bound
+    is 1e-3, each by one step."""
+    turns = [(0, 40), (40, 24)]
+    La, W, qw, kw, x, h0 = _setup(orc, dev, 77, 64, 8)
+    Lb = _setup(orc, dev, 77, 64, 8)[0]
+    xd = torch.from_numpy(x.view(np.int16)).to(dev).view(torch.float16)
+    h = torch.zeros((64, H), dtype=torch.float32, device=dev)
+    print("short turns beside single tokens", flush=True)
+    for s, n in turns:
+        La.block_forward(xd[s:s + n].contiguous(), h[s:s + n], s)
+    for s in range(64):
+        Lb.block_forward(xd[s:s + 1].contiguous(), h[s:s + 1], s)
+    torch.cuda.synchronize()
+    assert La.committed == Lb.committed == 64
+    for name in ("kc8", "vc8"):
+        a, b = (getattr(L, name)[:64].cpu().numpy().astype(np.int16) for L in (La, Lb))
+        d = np.abs(a - b)
+        assert d.max() <= 1 and (d > 0).mean() <= 1e-3, (name, d.max(), (d > 0).mean())
+    for name in ("ksc", "vsc"):
+        a, b = (getattr(L, name)[:1].cpu().numpy().view(np.int16).astype(np.int32) for L in (La, Lb))
+        assert np.abs(a - b).max() <= 2, name
