@@ -547,7 +547,8 @@ def main():
         f_qkv = 2.0 * S * H * (NH * D + 2 * NKV * D)
         f_o = 2.0 * S * H * NH * D
         prefill["int4_projections"] = {
-            "kernel": "k_gemm_int4 (v_mfma_f32_16x16x32_f16, exact nibble operands, "
+            "kernel": "INT4 matrix-core GEMM, tiles by the rows of x and W (4096 rows: "
+                      "k_gemm_int4_big; v_mfma_f32_16x16x32_f16, exact nibble operands, "
                       "per-group fp32 scaling)",
             "qkv_us": round(qkv_ms * 1e3, 1),
             "qkv_tflops": round(f_qkv / (qkv_ms * 1e-3) / 1e12, 1),

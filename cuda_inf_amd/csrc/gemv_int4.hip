@@ -447,8 +447,8 @@ __global__ __launch_bounds__(64 * kGemmWaves) void k_gemm_int4(GemvArgs a) {
 // next group's DMA goes out after the barrier that ends the last group and has
 // the whole step to land.  Layouts, the order of k and the sums are the tile
 // kernel's: the same bits.  K up to 2048 (the LDS).
-// (q/k/v of 4096 rows, kNT = 3, one round of 256 workgroups: 77 -> 58 us, 885
-// TFLOP/s; out_proj, kNT = 2: 66 -> 51.)
+// (q/k/v of 4096 rows, kNT = 3, one round of 256 workgroups: 77 us in 128 x 128
+// tiles, 55 so, 930 TFLOP/s; out_proj into the residual, kNT = 2: 69, 51.)
 constexpr int kBigRows = 256;
 
 // grid = the tiles, ceil(rows / (64 kNT)) * ceil(M / 256), up to a multiple of 8;
@@ -603,7 +603,7 @@ __global__ __launch_bounds__(64 * kGemmWaves) void k_gemm_int4_big(GemvArgs a) {
 }
 
 // ---------------------------------------------------------------- K-split GEMM
-// A few to about a thousand rows of x (short prompts, chat turns): too few
+// A few to some hundred rows of x (short prompts, chat turns): too few
 // 128 x 128 tiles to fill the chip, and each tile's 16 scale groups a serial
 // chain.  Here a workgroup computes a (16 kMT) x (16 kNT) tile with 8 waves
 // that split K: wave w takes the scale groups w, w + 8, .. (two of them at
@@ -630,9 +630,8 @@ __global__ __launch_bounds__(64 * kGemmWaves) void k_gemm_int4_big(GemvArgs a) {
 // are added in four chains a pass: the GEMV's sums are trees, and 16 roundings
 // in a row are further off (out_proj into the residual, 2-norm from 64 bits:
 // GEMV 7.2e-8, in order 7.65e-8, so 6.3e-8).
-// (Two passes at K = 2048.  out_proj of 300 rows, a call: 14.7 us with one
-// meeting of the waves' own scaled sums and all four k steps' x in registers,
-// 11.8 as here.)
+// (Two passes at K = 2048.  out_proj of 300 rows: 28.0 us in 128 x 128 tiles,
+// 10.8 so; 23 rows of q/k/v: 13.2 by the GEMV, 5.1 so.)
 constexpr int kKsWaves = 8;
 
 // grid = (ceil(rows / (16 kNT)), ceil(M / (16 kMT))), block = 512; K <= kKsMaxK

@@ -582,8 +582,9 @@ __global__ __launch_bounds__(1024) void k_h2o_mass(H2oArgs a, int nsw) {
 // Queries that see no slot of a block or workgroup are passed over; a product
 // of a slot that its query does not see is -0, which leaves any sum as it is.
 // (S = 1024 into an empty 2048-slot buffer: per 16 queries a scores and a mass
-// launch, its chain on one workgroup per 256 slots, 2500 us in all; as here 277.  By
-// the launch: stats 76, weights 7, chain 178, outputs 28.)
+// launch, its chain on one workgroup per 256 slots, 2500 us in all; as here 274.  By
+// the launch, in a kernel trace, whose times hold each launch's start: outputs 28.4,
+// stats 73.7, weights 6.7, chain 171.8, and 9.9 for the placement before them.)
 struct MassArgs {
   const uint16_t* q;  // first query row of the chunk
   const uint8_t* kf;
@@ -596,9 +597,9 @@ struct MassArgs {
 };
 // Queries from which these launches run instead of the pair per 16 queries: few
 // queries leave the chip idle in four launches where the pair is two.  (Pair /
-// these, us, attention over 2048 slots: S = 8 28 / 37, 16 50 / 41, 64 191 /
-// 68; a prompt into an empty buffer, with placement: 8 29 / 30, 16 47 / 36,
-// 64 136 / 37.)
+// these, us, attention over 2048 slots: S = 8 26 / 34, 16 48 / 37, 64 190 /
+// 63; over 64 slots: 8 19.2 / 19.7, 16 33 / 21, 64 127 / 29; over 4096: 16 62 /
+// 58.)
 constexpr int kManyMin = 16;
 constexpr int kStQ = 4;  // queries of a stats group
 
@@ -663,7 +664,7 @@ __global__ __launch_bounds__(256) void k_h2o_stats(MassArgs a, int ngrp) {
   // A q row is the same for every lane: it comes through the scalar cache into
   // 32 scalar registers, the next head's while this one's products are taken.
   // (Read back from LDS by every lane, a row's 8 reads of 1 KB were as much LDS
-  // time as the products' issue: 81 us in the prompt above, 76 so.)
+  // time as the products' issue: 81 us in the prompt above, 76 so, on one box.)
   u32x16 qs[2][2];
   auto load_q = [&](int n, u32x16 (&o)[2]) __attribute__((always_inline)) {  // head n of query i on
     const int in = min(i + (n >> 2), ie - 1);

@@ -415,8 +415,8 @@ int split_shape(const PrefillArgs& a, const SlotArgs& sl, int tiles, hipStream_t
 // x 64 key) tiles of all query heads, spread over every compute unit; the
 // block kernel's with the tiles of one workgroup (a heavy and a light block),
 // whether or not its 8 per pair of blocks fill the chip.  (Block / split: 77
-// queries at 0 11.9 / 4.8, 500 at 0 21.8 / 8.0, 2048 at 0 53.2 / 45.2, 77 at
-// 9000 314 / 25, 1000 at 8000 329 / 125; 4096 at 0 105 / 159.)
+// queries at 0 11.0 / 4.0, 500 at 0 20.6 / 7.5, 2048 at 0 52 / 46, 77 at 9000
+// 313 / 25, 1000 at 9000 361 / 151; 3000 at 0 70 / 96, 4096 at 0 91 / 154.)
 extern "C" __attribute__((visibility("hidden"))) int cia_prefill_split_wins(int S, int past) {
   const double tiles = (past + 0.5 * S) / 64.0 + 0.5;
   const double split = 4.0 + 1.15e-3 * NH * ((S + 31) / 32) * tiles;
