@@ -168,24 +168,32 @@ def test_kernels_have_the_tile_kernels_bits(orc, cia, dev, int4_choose, N, K, sh
                 assert torch.equal(z[:n], y[:n]) and not z.isnan().any(), (i, m)
 
 
-@pytest.mark.parametrize("N,K,seed", [(64, 2048, 70), (3072, 2048, 71), (8192, 2176, 72)])
-def test_few_rows_have_the_same_bits(orc, cia, dev, int4_choose, N, K, seed):
+@pytest.mark.parametrize("N,K,shapes,seed", [
+    (64, 2048, {0}, 70), (3072, 2048, {0, 1, 2}, 71), (9000, 2176, {1, 3, 4}, 72), (12300, 4096, {1, 2, 5}, 73)])
+def test_few_rows_have_the_same_bits(orc, cia, dev, int4_choose, N, K, shapes, seed):
     """Below 56 rows of x the sums take another order (four chains a pass), the
-    same in every tile shape: 55 rows against slices of them."""
+    same in every tile shape: 55 rows against slices of them, and against the
+    same rows of a narrow matrix (its own shapes)."""
     from cuda_inf_amd import kernels as KK
     rng = np.random.default_rng(seed)
     M, lo = 55, 3 + 2 * int4_choose([(3, N, K)])[0][1]
+    assert {c[0] for c in int4_choose([(m, N, K) for m in (lo, 16, 17, 33, 40, 55)])} == shapes
     packed, scales = _weights(rng, N, K, orc)
     xd = _t(rng.standard_normal((M, K)).astype(np.float16), dev)
     pd, sd = _t(packed, dev), _t(scales, dev)
-    y = torch.zeros((M, N), dtype=torch.float32, device=dev)
+    y = torch.full((M, N), float("nan"), dtype=torch.float32, device=dev)
     KK.gemv_int4(xd, pd, sd, y, N, K, M)
     for m in (lo, 16, 17, 33, 40):
-        z = torch.zeros((m, N), dtype=torch.float32, device=dev)
+        z = torch.full((m, N), float("nan"), dtype=torch.float32, device=dev)
         print(f"N={N} K={K} M={m}", flush=True)
         KK.gemv_int4(xd[:m], pd, sd, z, N, K, m)
         torch.cuda.synchronize()
         assert torch.equal(z, y[:m]), m
+    n = 40  # the first 40 rows of W alone
+    z = torch.full((M, n), float("nan"), dtype=torch.float32, device=dev)
+    KK.gemv_int4(xd, pd, sd, z, n, K, M)
+    torch.cuda.synchronize()
+    assert torch.equal(z, y[:, :n])
 
 
 # The 256-row tiles: 128 and 192 columns a tile, each with ragged last rows and
