@@ -18,12 +18,19 @@ from ._lib import D, KVGROUP, NH, NKV, NSPLIT_DEFAULT, call
 _F16 = (torch.float16, torch.int16, torch.uint16)
 
 
+# torch's own short way to the current stream's handle; no public name, so a
+# build of torch without it takes the long way
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_handle() -> int:
     """The hipStream_t of torch's current stream on the current device: the
     value of ``torch.cuda.current_stream().cuda_stream`` without the stream
     object (2.8 -> 0.3 us, of an 8.3 us gemv_int4 call of one row, whose
     kernel takes 2.9).  Read on every call, like that one."""
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
 
 
 def _dev(t: torch.Tensor, name: str, dtypes=None, numel=None):

@@ -186,3 +186,18 @@ def test_h2o_pick_matches_oracle(cia, orc):
         b = orc.h2o_pick_slots(n_live, C, W, sp.copy(), at.copy(), S, past)
         assert a[0] == b[0] and np.array_equal(a[1], b[1]) and np.array_equal(a[2], b[2]) \
             and a[3] == b[3]
+
+
+def test_stream_handle_without_torchs_short_way(monkeypatch):
+    """A build of torch without the private accessor of the current stream's
+    handle: the public one is used."""
+    import importlib
+    import types
+    import torch
+    from cuda_inf_amd import kernels
+    with monkeypatch.context() as m:
+        m.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+        m.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=77))
+        importlib.reload(kernels)
+        assert kernels.stream_handle() == 77
+    importlib.reload(kernels)
